@@ -485,6 +485,9 @@ def _extended_loss(*, x, weight, labels, teacher, norm: StudentRMSNorm | None, f
         ignore_index=int(kw["ignore_index"]), reduction=kw["reduction"], divergence=divergence,
         token_chunk=int(cs), eps=eps, fp8_logits=fp8,
     )
+    from .ops._engine import without_autograd
+
+    x, nw, weight, t_hidden, t_weight = without_autograd(x, nw, weight, t_hidden, t_weight)
     out = RMSNormPrologueFunction.apply(x, nw, weight, t_hidden, t_weight, labels, spec)
     return DistillationLossOutput(*out)
 

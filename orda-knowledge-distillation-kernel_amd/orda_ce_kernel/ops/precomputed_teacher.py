@@ -20,7 +20,7 @@ from .._runtime import default_compute_dtype
 from ..utils.resolver import DEFAULT_MAX_FUSED_SIZE
 from ._checks import check_common, check_labels_in_range, check_scalars
 from ._engine import (FusedCall, cast_to, fused_backward, fused_forward, grads_in_forward, require_native,
-                      token_chunk_for, vocab_chunk_for)
+                      token_chunk_for, vocab_chunk_for, without_autograd)
 
 __all__ = ["PrecomputedCEFunction", "precomputed_distillation_loss"]
 
@@ -221,6 +221,7 @@ def precomputed_distillation_loss(
     _check_devices(student_hidden, labels, weight, logits_teacher, teacher_hidden, teacher_weight)
     if validate_labels:
         check_labels_in_range(labels, V, ignore_index)
+    student_hidden, weight = without_autograd(student_hidden, weight)
     return PrecomputedCEFunction.apply(
         student_hidden, weight, logits_teacher, labels, student_ce_weight, ignore_index, reduction, chunk_size,
         use_fp32_accum, kl_weight, kl_temperature, w_t, max_chunks, max_fused_size, autotune, teacher_hidden,
@@ -247,6 +248,7 @@ def precomputed_distillation_loss_with_teacher_ce(
     _check_devices(student_hidden, labels, weight, logits_teacher, teacher_hidden, teacher_weight)
     if validate_labels:
         check_labels_in_range(labels, V, ignore_index)
+    student_hidden, weight = without_autograd(student_hidden, weight)
     return PrecomputedTeacherCEFunction.apply(
         student_hidden, weight, logits_teacher, labels, student_ce_weight, ignore_index, reduction, chunk_size,
         use_fp32_accum, kl_weight, kl_temperature, w_t, max_chunks, max_fused_size, autotune, teacher_hidden,

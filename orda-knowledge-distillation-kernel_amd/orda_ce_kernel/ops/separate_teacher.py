@@ -17,7 +17,7 @@ from .._runtime import default_compute_dtype
 from ..utils.resolver import DEFAULT_MAX_FUSED_SIZE
 from ._checks import check_common, check_labels_in_range, check_scalars
 from ._engine import (FusedCall, cast_to, fused_backward, fused_forward, grads_in_forward, require_native,
-                      token_chunk_for, vocab_chunk_for)
+                      token_chunk_for, vocab_chunk_for, without_autograd)
 
 __all__ = ["SeparateFullCEFunction", "SeparateStudentCEFunction", "separate_distillation_loss"]
 
@@ -218,6 +218,8 @@ def separate_distillation_loss(
     if validate_labels:
         check_labels_in_range(labels, V, ignore_index)
     function = SeparateFullCEFunction if w_t > 0.0 else SeparateStudentCEFunction
+    student_hidden, teacher_hidden, weight, teacher_weight = without_autograd(
+        student_hidden, teacher_hidden, weight, teacher_weight)
     return function.apply(
         student_hidden, teacher_hidden, weight, teacher_weight, labels, student_ce_weight, ignore_index,
         reduction, chunk_size, use_fp32_accum, kl_weight, kl_temperature, w_t, max_chunks, max_fused_size,

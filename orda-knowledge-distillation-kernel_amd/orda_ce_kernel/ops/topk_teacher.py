@@ -32,7 +32,7 @@ from .._runtime import default_compute_dtype
 from ..divergences import resolve_divergence
 from ..utils.resolver import DEFAULT_MAX_FUSED_SIZE
 from ._checks import check_common, check_labels_in_range, check_scalars
-from ._engine import FusedCall, cast_to, fused_backward, fused_forward, require_native, token_chunk_for
+from ._engine import FusedCall, cast_to, fused_backward, fused_forward, require_native, token_chunk_for, without_autograd
 
 __all__ = ["TOPK_DIVERGENCES", "TopKCEFunction", "check_topk_teacher", "topk_distillation_loss"]
 
@@ -156,6 +156,7 @@ def topk_distillation_loss(
         raise ValueError(f"tensors must be CUDA/HIP tensors, got device={device}")
     if validate_labels:
         check_labels_in_range(labels, V, ignore_index)
+    student_hidden, weight = without_autograd(student_hidden, weight)
     return TopKCEFunction.apply(
         student_hidden, weight, topk_indices, topk_logprobs, labels, student_ce_weight, ignore_index, reduction,
         chunk_size, kl_weight, kl_temperature, max_chunks, max_fused_size, divergence,
