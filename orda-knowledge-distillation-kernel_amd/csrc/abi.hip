@@ -713,17 +713,12 @@ int run_backward(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* 
   // Transposed hidden states for the grad_W GEMMs (K = tokens), with zeroed
   // padding columns so K can be rounded up to a multiple of 8.
   if (pl.need_gw) {
-    { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(hT, pl.ldh, H, N, NP, eb, s)); }
-    { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(t->student_hidden, H, hT, pl.ldh, N, H, s)); }
-    if (tied && pl.w_dlt_t) {
-      { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(hT, pl.ldh, H, NP + N, 2 * NP, eb, s)); }
-      { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(t->teacher_hidden, H, hT + NP * eb, pl.ldh, N, H, s)); }
-    }
+    { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(t->student_hidden, H, hT, pl.ldh, N, NP, H, s)); }
+    if (tied && pl.w_dlt_t)
+      { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(t->teacher_hidden, H, hT + NP * eb, pl.ldh, N, NP, H, s)); }
   }
-  if (sep && pl.w_dlt_t) {
-    { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(htT, NP, Ht, N, NP, eb, s)); }
-    { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(t->teacher_hidden, Ht, htT, NP, N, Ht, s)); }
-  }
+  if (sep && pl.w_dlt_t)
+    { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(t->teacher_hidden, Ht, htT, NP, N, NP, Ht, s)); }
   // padding columns of the staged dlogits (never written by the dL kernel)
   if (pl.w_dlt_s || pl.w_dlt_t) { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(dLT, pl.ldT, pl.Vc, N, NP, eb, s)); }
   if (pl.w_dlt_t) { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(dLT, pl.ldT, pl.Vc, NP + N, 2 * NP, eb, s)); }
@@ -756,12 +751,10 @@ int run_backward(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* 
                       : c == pl.nchunks - 1 ? GEMM_ACC_LAST : GEMM_ACC;
     const bool needWT = pl.need_gs || (tied && pl.w_dln_t);
     if (needWT) {
-      { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(static_cast<const char*>(t->weight) + vc0 * H * eb, H, WT, pl.Vc, vcc, H, s)); }
-      if (vck > vcc) { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(WT, pl.Vc, H, vcc, vck, eb, s)); }
+      { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(static_cast<const char*>(t->weight) + vc0 * H * eb, H, WT, pl.Vc, vcc, vck, H, s)); }
     }
     if (sep && pl.w_dln_t) {
-      { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(static_cast<const char*>(t->teacher_weight) + vc0 * Ht * eb, Ht, WtT, pl.Vc, vcc, Ht, s)); }
-      if (vck > vcc) { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(WtT, pl.Vc, Ht, vcc, vck, eb, s)); }
+      { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(static_cast<const char*>(t->teacher_weight) + vc0 * Ht * eb, Ht, WtT, pl.Vc, vcc, vck, Ht, s)); }
     }
     if (vck > vcc) {
       if (pl.w_dln_s) { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(dLNs, pl.Vc, N, vcc, vck, eb, s)); }
@@ -827,6 +820,20 @@ int gemm2(int la, int lb, const void* A, int64_t lda, const void* B, int64_t ldb
   return ORDA_OK;
 }
 
+// k_dlm's launch: its waves beside each other as far as the chunk's 256-token
+// groups reach, and 64 rows per wave (whose row parameters cost 16 loads),
+// fewer (down to 16) while the launch has under 4096 waves, 4 per SIMD: the
+// stream needs that many in flight.
+inline void dlm_shape(DlmParams& D) {
+  const int64_t groups = cdiv(D.Npad, 256);
+  D.wave_cols = groups >= 3 ? 4 : (groups == 2 ? 2 : 1);
+  int64_t rows = 64;
+  while (rows > 16 && groups * cdiv(D.V, rows) < 4096) rows /= 2;
+  const int64_t below = 4 / D.wave_cols;
+  rows = std::max<int64_t>(rows, cdiv(D.V, 65535 * below));  // grid.y stays <= 65535
+  D.rows_per_block = (int)round_up(rows, 8);
+}
+
 // Forward with the gradients (ORDA_GRADS_IN_FORWARD), token chunk by token
 // chunk: label logits, the scan with the logits stored vocabulary-major in L,
 // the per-row merge, dlogits in place (k_dlm), grad W += dL^T [hs; ht]
@@ -836,7 +843,7 @@ template <class T>
 int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, char* ws, hipStream_t s) {
   const bool tied = pl.mode == ORDA_MODE_TIED, sep = pl.mode == ORDA_MODE_SEPARATE;
   const int eb = pl.eb;
-  const int64_t N = pl.N, V = pl.V, H = pl.H, Ht = pl.Ht, nP = pl.fnP, ldL = pl.fldL;
+  const int64_t N = pl.N, V = pl.V, H = pl.H, Ht = pl.Ht, ldL = pl.fldL;
   char* L = ws + pl.off_L;
   float* part = reinterpret_cast<float*>(ws + pl.off_fpart);
   float* labelx = reinterpret_cast<float*>(ws + pl.off_flabelx);
@@ -870,6 +877,10 @@ int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, 
   for (int64_t c = 0; c < pl.fnchunks; ++c) {
     const int64_t r0 = c * pl.fn;
     const int64_t nc = (N - r0 < pl.fn) ? N - r0 : pl.fn;
+    // the chunk's token columns in L and hT, padded: a short last chunk
+    // packs its student and teacher columns side by side too, so grad W's K
+    // is its own token count
+    const int64_t nP = round_up(nc, 8);
 
     // the chunk's student rows as the GEMMs see them: the caller's, or their
     // RMSNorm (then x is the caller's rows and hsc the normalised copy)
@@ -948,7 +959,7 @@ int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, 
         F.tsrc = TSRC_MEM_RING;
       } else if (pl.tsrc == TSRC_MEM && same_dtype) {
         Timed tm_(ORDA_K_AUX, s, 0.0, 0.0);
-        ORDA_CHECK_LAUNCH(launch_transpose<T>(Ltc, V, Lt, ldL, nc, V, s));
+        ORDA_CHECK_LAUNCH(launch_transpose<T>(Ltc, V, Lt, ldL, nc, nc, V, s));
       } else if (pl.tsrc == TSRC_MEM) {
         // logits of another dtype: cast to the compute dtype on the way into
         // L, as the reference casts each chunk (ops/precomputed_teacher.py:343-348)
@@ -1027,9 +1038,9 @@ int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, 
 
     DlmParams D{};
     D.L = L; D.ldL = ldL; D.tcol = nP; D.labels = t->labels + r0; D.rowp = rowp; D.mean_scale = pl.late_scale ? scal + 2 : scal;
-    D.N = nc; D.V = V; D.ignore_index = p->ignore_index;
+    D.N = nc; D.Npad = nP; D.V = V; D.ignore_index = p->ignore_index;
     D.div = pl.div; D.t_is_one = pl.t1; D.tgrad = tgrad;
-    D.rows_per_block = (int)round_up(std::max<int64_t>(64, cdiv(V, 65535)), 8);  // grid.y stays <= 65535
+    dlm_shape(D);
     D.Ltm = pl.f_tmem ? Ltc : nullptr;
     D.ldtm = V;
     D.invT = F.invT; D.temperature = p->temperature; D.alpha = p->div_alpha; D.beta = p->div_beta;
@@ -1038,19 +1049,11 @@ int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, 
     { Timed tm_(ORDA_K_DLOGITS, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_dlm<T>(D, s)); }
     if (pl.topk && pl.div_on) { Timed tm_(ORDA_K_DLOGITS, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_topk_scatter<T>(K, s)); }
 
-    // token columns [nc, nP) of L are read by the grad-W GEMM (K = tokens):
-    // keep them zero (the matching hidden rows read as zero too)
-    if (nc < nP) {
-      { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(L, ldL, V, nc, nP, eb, s)); }
-      if (pl.store_t) { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(L, ldL, V, nP + nc, 2 * nP, eb, s)); }
-    }
-
     // grad W (+)= dL^T [hs; ht] with both operands K-major over tokens: the
     // chunk's hidden states are transposed into hT (padding columns zero)
     const int wmode = c == 0 ? GEMM_STORE : GEMM_ACC_T;
     auto transpose_chunk = [&](const T* src, int64_t cols, char* dst, int64_t ldd, int64_t col0) -> int {
-      { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(src, cols, dst + col0 * eb, ldd, nc, cols, s)); }
-      if (nc < nP) { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(dst, ldd, cols, col0 + nc, col0 + nP, eb, s)); }
+      { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(src, cols, dst + col0 * eb, ldd, nc, nP, cols, s)); }
       return ORDA_OK;
     };
     if (pl.need_gw) {

@@ -2039,26 +2039,16 @@ struct TmTile {
   }
 };
 
-// 4 consecutive elements as raw bits (one 8- or 16-byte load when n == 4;
-// elements past n read as zero bits), converted to fp32 at their use: the
-// streaming passes keep a 16-bit row in two registers instead of four.
+// 4 consecutive elements as raw bits (one 8- or 16-byte load), converted to
+// fp32 at their use: the streaming passes keep a 16-bit row in two registers
+// instead of four.  L's columns are padded to a multiple of 8 tokens, so a
+// quad that straddles the last token is loaded whole too (its padding columns
+// hold anything until the dlogits pass zeroes them).
 template <class T> struct Raw4 { typedef uint2 type; };
 template <> struct Raw4<float> { typedef uint4 type; };
 template <class T>
-__device__ __forceinline__ typename Raw4<T>::type load_raw4(const T* p, int n) {
-  if constexpr (sizeof(T) == 2) {
-    if (n == 4) return *reinterpret_cast<const uint2*>(p);
-    uint32_t e[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) e[i] = i < n ? (uint32_t)__builtin_bit_cast(unsigned short, p[i]) : 0u;
-    return make_uint2(e[0] | (e[1] << 16), e[2] | (e[3] << 16));
-  } else {
-    if (n == 4) return *reinterpret_cast<const uint4*>(p);
-    uint32_t e[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) e[i] = i < n ? __float_as_uint(p[i]) : 0u;
-    return make_uint4(e[0], e[1], e[2], e[3]);
-  }
+__device__ __forceinline__ typename Raw4<T>::type load_raw4(const T* p) {
+  return *reinterpret_cast<const typename Raw4<T>::type*>(p);
 }
 template <class T>
 __device__ __forceinline__ void unpack4(const typename Raw4<T>::type& u, float (&x)[4]) {
@@ -2127,8 +2117,8 @@ __global__ __launch_bounds__(256) void k_two_rows(TwoParams P) {
     auto load_rows = [&](int64_t vv) {
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        xs[r] = load_raw4(Ls + (vv + 4 * r) * P.ldL, nt);
-        xt[r] = load_raw4(Lt + (vv + 4 * r) * P.ldL, nt);
+        xs[r] = load_raw4(Ls + (vv + 4 * r) * P.ldL);
+        xt[r] = load_raw4(Lt + (vv + 4 * r) * P.ldL);
       }
     };
     if (v + 4 * (R - 1) < v1) load_rows(v);
@@ -2143,7 +2133,7 @@ __global__ __launch_bounds__(256) void k_two_rows(TwoParams P) {
 #pragma unroll
       for (int r = 0; r < R; ++r) rows(cs[r], ct[r]);
     }
-    for (; v < v1; v += 4) rows(load_raw4(Ls + v * P.ldL, nt), load_raw4(Lt + v * P.ldL, nt));
+    for (; v < v1; v += 4) rows(load_raw4(Ls + v * P.ldL), load_raw4(Lt + v * P.ldL));
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -2211,7 +2201,7 @@ __global__ __launch_bounds__(256) void k_two_rows_tm(TwoParams P) {
       for (int m = 0; m < M; ++m) {
         const int64_t v = vb + w + 4 * m;
         xs[m] = {};
-        if (nt > 0 && v < v1) xs[m] = load_raw4(Ls + v * P.ldL, nt);
+        if (nt > 0 && v < v1) xs[m] = load_raw4(Ls + v * P.ldL);
       }
     }
   };
@@ -2258,10 +2248,11 @@ __global__ __launch_bounds__(256) void k_two_rows_tm(TwoParams P) {
 // Row parameters of 4 consecutive tokens and their dlogits for one
 // vocabulary row: student w_s (p_s - 1_y) + w_kl T dD/dz_s, teacher
 // w_t (p_t - 1_y), times mean_scale (the caller's grad_output is applied
-// later); ignored tokens (and tokens past the quad's nt) give 0.
+// later); ignored tokens give 0, and so do tokens past the quad's nt after
+// clip() (their logits are padding: anything, NaN included).
 template <int DIV, bool T1>
 struct DlmQuad {
-  int64_t yeff[4];
+  int yeff[4];
   float lse_s[4], lse_sT[4], lse_t[4], lse_tT[4], c[4][4], sc_s[4], sc_t[4], sc_d[4];
   float invT, alpha, beta;
 
@@ -2276,7 +2267,7 @@ struct DlmQuad {
       const int64_t t = t0 + (ok ? i : 0);
       const int64_t y = P.labels[t];
       const bool ign = !ok || y == P.ignore_index;
-      yeff[i] = (y >= 0 && y < P.V) ? y : 0;
+      yeff[i] = (y >= 0 && y < P.V) ? (int)y : 0;  // (V <= 2^30)
       lse_s[i] = P.rowp[0 * P.N + t];
       lse_sT[i] = P.rowp[1 * P.N + t];
       lse_t[i] = P.rowp[2 * P.N + t];
@@ -2288,7 +2279,11 @@ struct DlmQuad {
       sc_d[i] = ign ? 0.f : scale * P.w_kl * P.temperature;
     }
   }
-  __device__ __forceinline__ void row(int64_t v, const float (&xs)[4], const float (&xt)[4], float (&ds)[4],
+  __device__ __forceinline__ static void clip(float (&d)[4], int nt) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d[i] = i < nt ? d[i] : 0.f;
+  }
+  __device__ __forceinline__ void row(int v, const float (&xs)[4], const float (&xt)[4], float (&ds)[4],
                                       float (&dt)[4]) const {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -2310,33 +2305,43 @@ struct DlmQuad {
 
 // In place on the logits L[v][t] of one token chunk (vocabulary-major,
 // student columns [0, N), teacher columns [tcol, tcol + N)): the dlogits of
-// DlmQuad.  Thread: 4 consecutive tokens x rows_per_block vocabulary rows;
-// block: 256 threads = 1024 tokens.
+// DlmQuad, and zeros in the padding columns [N, Npad) that the grad-W GEMM
+// reads (K = tokens).  A wave takes 256 tokens (a lane's 4 consecutive) x
+// rows_per_block rows; the block's 4 waves lie `wave_cols` beside each other
+// along the tokens and 4 / wave_cols below each other (a 256-token chunk
+// would leave three waves of a 1024-token block idle).  The wave that holds
+// the chunk's last, partial quad runs the same batched loop with its lanes'
+// outputs clipped: a per-element path for that one lane took 64 rows of
+// dependent scalar loads (the call at 1999 tokens, hidden 768, vocabulary
+// 50257, T = 2: 1177 us, 1062 without it).
 template <class T, int DIV, bool T1, bool NO_T = false>
 __global__ __launch_bounds__(256) void k_dlm(DlmParams P) {
-  const int64_t t0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
-  if (t0 >= P.N) return;
-  const int nt = (int)min<int64_t>(P.N - t0, 4);
-  const int64_t v0 = (int64_t)blockIdx.y * P.rows_per_block;
-  const int64_t v1 = min<int64_t>(P.V, v0 + P.rows_per_block);
+  const int w = wave_id();
+  const int wx = w % P.wave_cols, wy = w / P.wave_cols;
+  const int64_t t0 = (((int64_t)blockIdx.x * P.wave_cols + wx) * 64 + (threadIdx.x & 63)) * 4;
+  if (t0 >= P.Npad) return;
+  const int nt = (int)max<int64_t>(0, min<int64_t>(P.N - t0, 4));
+  const int v0 = (int)(((int64_t)blockIdx.y * (4 / P.wave_cols) + wy) * P.rows_per_block);
+  const int v1 = (int)min<int64_t>(P.V, (int64_t)v0 + P.rows_per_block);
+  if (v0 >= v1) return;
   DlmQuad<DIV, T1> q;
-  q.init(P, t0, nt);
+  q.init(P, nt > 0 ? t0 : 0, nt);
   T* Ls = static_cast<T*>(P.L) + t0;
   T* Lt = Ls + P.tcol;
   // (a compile-time no-teacher variant: a run-time flag here splits the
   // interior loop's batched loads)
   const bool need_t = !NO_T && (DIV >= 0 || P.tgrad);
-  int64_t v = v0;
-  if (nt == 4) {
-    // interior: R rows per iteration, every load issued before any use
+  using Raw = typename Raw4<T>::type;
+  int v = v0;
+  auto rows = [&](auto clipped) {
+    // R rows per iteration, every load issued before any use
     constexpr int R = 8;
-    using Raw = typename Raw4<T>::type;
     for (; v + R <= v1; v += R) {
       Raw us[R], ut[R];
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        us[r] = load_raw4(Ls + (v + r) * P.ldL, 4);
-        ut[r] = need_t ? load_raw4(Lt + (v + r) * P.ldL, 4) : Raw{};
+        us[r] = load_raw4(Ls + (int64_t)(v + r) * P.ldL);
+        ut[r] = need_t ? load_raw4(Lt + (int64_t)(v + r) * P.ldL) : Raw{};
       }
 #pragma unroll
       for (int r = 0; r < R; ++r) {
@@ -2344,19 +2349,26 @@ __global__ __launch_bounds__(256) void k_dlm(DlmParams P) {
         unpack4<T>(us[r], xs);
         unpack4<T>(ut[r], xt);
         q.row(v + r, xs, xt, ds, dt);
-        store4(Ls + (v + r) * P.ldL, ds, true, 4);
-        if (P.tgrad) store4(Lt + (v + r) * P.ldL, dt, true, 4);
+        if constexpr (decltype(clipped)::value) {
+          q.clip(ds, nt);
+          q.clip(dt, nt);
+        }
+        store4(Ls + (int64_t)(v + r) * P.ldL, ds, true, 4);
+        if (P.tgrad) store4(Lt + (int64_t)(v + r) * P.ldL, dt, true, 4);
       }
     }
-  }
-  // edges: the last rows of the block, or a partial token quad
-  for (; v < v1; ++v) {
-    float xs[4], xt[4] = {0.f, 0.f, 0.f, 0.f}, ds[4], dt[4];
-    load4(Ls + v * P.ldL, xs, nt == 4, nt);
-    if (need_t) load4(Lt + v * P.ldL, xt, nt == 4, nt);
+  };
+  if (__all(nt == 4)) rows(std::false_type{});
+  else rows(std::true_type{});
+  for (; v < v1; ++v) {  // the last rows of the vocabulary
+    float xs[4], xt[4], ds[4], dt[4];
+    unpack4<T>(load_raw4(Ls + (int64_t)v * P.ldL), xs);
+    unpack4<T>(need_t ? load_raw4(Lt + (int64_t)v * P.ldL) : Raw{}, xt);
     q.row(v, xs, xt, ds, dt);
-    store4(Ls + v * P.ldL, ds, nt == 4, nt);
-    if (P.tgrad) store4(Lt + v * P.ldL, dt, nt == 4, nt);
+    q.clip(ds, nt);
+    q.clip(dt, nt);
+    store4(Ls + (int64_t)v * P.ldL, ds, true, 4);
+    if (P.tgrad) store4(Lt + (int64_t)v * P.ldL, dt, true, 4);
   }
 }
 
@@ -2381,7 +2393,7 @@ __global__ __launch_bounds__(256) void k_dlm_tm(DlmParams P) {
   const int64_t t0 = tb + lane * 4;
   const int64_t rem = P.N - t0;
   const int nt = rem <= 0 ? 0 : (rem >= 4 ? 4 : (int)rem);
-  const bool live = nt > 0;
+  const bool live = t0 < P.Npad;  // (padding quads write zeros)
   const bool interior = tb + kTmTok <= P.N && v0 + kTmRows <= P.V;  // block-uniform
   T* Ls = static_cast<T*>(P.L) + (live ? t0 : 0);
   constexpr int M = kTmRows / 4;  // rows per wave
@@ -2400,11 +2412,11 @@ __global__ __launch_bounds__(256) void k_dlm_tm(DlmParams P) {
     for (int m = 0; m < M; ++m) {
       const int64_t v = v0 + w + 4 * m;
       xs[m] = {};
-      if (live && v < P.V) xs[m] = load_raw4(Ls + v * P.ldL, nt);
+      if (live && v < P.V) xs[m] = load_raw4(Ls + v * P.ldL);
     }
   }
   DlmQuad<DIV, T1> q;
-  q.init(P, live ? t0 : 0, nt);
+  q.init(P, nt > 0 ? t0 : 0, nt);
   tm.put(tile);
   __syncthreads();
   if (!live) return;
@@ -2416,7 +2428,7 @@ __global__ __launch_bounds__(256) void k_dlm_tm(DlmParams P) {
       float x[4], xt[4], ds[4], dt[4];
       unpack4<T>(xs[m], x);
       TmTile<T>::read(tile, lane, r, xt);
-      q.row(v0 + r, x, xt, ds, dt);
+      q.row((int)v0 + r, x, xt, ds, dt);
       *reinterpret_cast<uint2*>(p) = make_uint2(pack2<T>(ds[0], ds[1]), pack2<T>(ds[2], ds[3]));
       p += step;
     }
@@ -2430,20 +2442,23 @@ __global__ __launch_bounds__(256) void k_dlm_tm(DlmParams P) {
     float x[4], xt[4], ds[4], dt[4];
     unpack4<T>(xs[m], x);
     TmTile<T>::read(tile, lane, r, xt);
-    q.row(v, x, xt, ds, dt);
-    store4(Ls + v * P.ldL, ds, nt == 4, nt);
+    q.row((int)v, x, xt, ds, dt);
+    q.clip(ds, nt);
+    store4(Ls + v * P.ldL, ds, true, 4);
   }
 }
 
 // ---------------------------------------------------------------- transpose
-// out[c * ldo + r] = in[r * ldi + c] for r < R, c < C (64 x 64 LDS tiles).
+// out[c * ldo + r] = in[r * ldi + c] for r < R, c < C (64 x 64 LDS tiles), and
+// zeros for r in [R, Rp) (the padding a K-major consumer reads).
 // 16-bit tiles wholly inside [0, R) x [0, C) with 16-byte aligned rows on
 // both sides (vec) move 16 bytes per access: thread -> rows tid / 8 and
 // tid / 8 + 32, piece tid % 8 (8 columns) on the way in; output rows the same
 // on the way out, each piece gathered from 8 tile rows.
 template <class T>
 __global__ __launch_bounds__(256) void k_transpose(const T* __restrict__ in, int64_t ldi, T* __restrict__ out,
-                                                   int64_t ldo, int64_t R, int64_t C, int tiles_c, int vec) {
+                                                   int64_t ldo, int64_t R, int64_t Rp, int64_t C, int tiles_c,
+                                                   int vec) {
   __shared__ __align__(16) T tile[64][72];  // (pitch 144 bytes: 16-byte aligned rows)
   const int tr = blockIdx.x / tiles_c, tc = blockIdx.x % tiles_c;
   const int64_t r0 = (int64_t)tr * 64, c0 = (int64_t)tc * 64;
@@ -2474,12 +2489,12 @@ __global__ __launch_bounds__(256) void k_transpose(const T* __restrict__ in, int
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
   for (int i = ty; i < 64; i += 4) {
     const int64_t r = r0 + i, c = c0 + tx;
-    if (r < R && c < C) tile[i][tx] = in[r * ldi + c];
+    tile[i][tx] = r < R && c < C ? in[r * ldi + c] : from_f32<T>(0.f);
   }
   __syncthreads();
   for (int i = ty; i < 64; i += 4) {
     const int64_t c = c0 + i, r = r0 + tx;
-    if (r < R && c < C) out[c * ldo + r] = tile[tx][i];
+    if (r < Rp && c < C) out[c * ldo + r] = tile[tx][i];
   }
 }
 
@@ -2768,13 +2783,13 @@ hipError_t launch_gemm(const GemmParams& P, hipStream_t s) {
   return hipGetLastError();
 }
 template <class T>
-hipError_t launch_transpose(const void* in, int64_t ldi, void* out, int64_t ldo, int64_t R, int64_t C,
+hipError_t launch_transpose(const void* in, int64_t ldi, void* out, int64_t ldo, int64_t R, int64_t Rp, int64_t C,
                             hipStream_t s) {
-  const int tiles_r = (int)((R + 63) / 64), tiles_c = (int)((C + 63) / 64);
+  const int tiles_r = (int)((Rp + 63) / 64), tiles_c = (int)((C + 63) / 64);
   const int vec = sizeof(T) == 2 && ldi % 8 == 0 && ldo % 8 == 0 && reinterpret_cast<uintptr_t>(in) % 16 == 0 &&
                   reinterpret_cast<uintptr_t>(out) % 16 == 0;
   hipLaunchKernelGGL(k_transpose<T>, dim3(tiles_r * tiles_c), dim3(256), 0, s, static_cast<const T*>(in), ldi,
-                     static_cast<T*>(out), ldo, R, C, tiles_c, vec);
+                     static_cast<T*>(out), ldo, R, Rp, C, tiles_c, vec);
   return hipGetLastError();
 }
 
@@ -3226,7 +3241,8 @@ inline void dlm_go(const DlmParams& P, hipStream_t s) {
       return;
     }
   }
-  const dim3 grid((unsigned)((P.N + 1023) / 1024), (unsigned)((P.V + P.rows_per_block - 1) / P.rows_per_block));
+  const int64_t cols = 256 * P.wave_cols, rows = (int64_t)(4 / P.wave_cols) * P.rows_per_block;
+  const dim3 grid((unsigned)((P.Npad + cols - 1) / cols), (unsigned)((P.V + rows - 1) / rows));
   hipLaunchKernelGGL((k_dlm<T, DIV, T1, NO_T>), grid, dim3(256), 0, s, P);
 }
 #define ORDA_DLM_CASE(T, D) \
@@ -3368,7 +3384,7 @@ inline void dlm_go(const DlmParams& P, hipStream_t s) {
 #define ORDA_INSTANTIATE_GEMM(T)                                                                     \
   template hipError_t launch_gemm<T>(const GemmParams&, hipStream_t);                                \
   template hipError_t launch_label<T>(const LabelParams&, hipStream_t);                              \
-  template hipError_t launch_transpose<T>(const void*, int64_t, void*, int64_t, int64_t, int64_t,    \
+  template hipError_t launch_transpose<T>(const void*, int64_t, void*, int64_t, int64_t, int64_t, int64_t, \
                                           hipStream_t);                                              \
   template hipError_t launch_transpose_cast<T>(const void*, int, int64_t, void*, int64_t, int64_t, int64_t, \
                                                hipStream_t);

@@ -101,10 +101,14 @@ struct DlmParams {
   const float* rowp;        // [kNRowP][N]
   const float* mean_scale;  // device scalar
   int64_t N, V, ignore_index;
-  int div, t_is_one, tgrad, rows_per_block;
+  int64_t Npad;  // columns [N, Npad) get zeros (Npad a multiple of 4, <= the padding of L's halves)
+  int div, t_is_one, tgrad;
+  // k_dlm: vocabulary rows per wave, and the block's waves beside each other
+  // along the tokens (1, 2 or 4)
+  int rows_per_block, wave_cols;
   float invT, temperature, alpha, beta, w_s, w_t, w_kl;
   // precomputed teacher logits read in place, token-major [N][ldtm] (16-byte
-  // aligned rows, ldtm a multiple of 8, rows_per_block a multiple of 8), when
+  // aligned rows, ldtm a multiple of 8), when
   // they are not staged in L's teacher columns; else null
   const void* Ltm;
   int64_t ldtm;
@@ -217,8 +221,9 @@ template <class T>
 hipError_t launch_splitk_reduce(const float* part, int splits, int64_t stride, void* out, int64_t ldo, int64_t M,
                                 int64_t N, hipStream_t s);
 template <class T> hipError_t launch_scale(void* x, int64_t n, const float* g, hipStream_t s);
+// out[c * ldo + r] = r < R ? in[r * ldi + c] : 0 for r < Rp, c < C
 template <class T>
-hipError_t launch_transpose(const void* in, int64_t ldi, void* out, int64_t ldo, int64_t R, int64_t C,
+hipError_t launch_transpose(const void* in, int64_t ldi, void* out, int64_t ldo, int64_t R, int64_t Rp, int64_t C,
                             hipStream_t s);
 // The same for logits of dtype in_dtype (DT_*), rounded once to T.
 template <class T>
