@@ -82,7 +82,7 @@ struct Plan {
   int tsrc, div, fam, npow;
   float pa[3], pb[3];
   // forward
-  int n_ttiles, n_vtiles, n_vranges, tiles_per_range;
+  int f_tok, n_ttiles, n_vtiles, n_vranges, tiles_per_range;
   size_t off_partial, off_labelx, off_rowv, fwd_bytes;
   size_t saved_bytes;
   // backward
@@ -276,10 +276,12 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
     }
   }
 
-  // forward plan
-  pl.n_ttiles = (int)cdiv(pl.N, 128);
+  // forward plan.  Scan tiles of 256 vocabulary rows x 128 tokens; fp32: 64
+  // tokens when the tile also holds a teacher's GEMM.
+  const bool f32 = p->dtype == ORDA_F32;
+  pl.n_ttiles = (int)cdiv(pl.N, f32 && (pl.tsrc == TSRC_SHARED || pl.tsrc == TSRC_SEP) ? 64 : 128);
   pl.n_vtiles = (int)cdiv(pl.V, 256);
-  int64_t nvr = cdiv(kScanTargetGroups, pl.n_ttiles);  // two-phase scan
+  int64_t nvr = f32 ? kPersistentGroups / pl.n_ttiles : cdiv(kScanTargetGroups, pl.n_ttiles);  // two-phase scan
   if (nvr < 1) nvr = 1;
   if (nvr > pl.n_vtiles) nvr = pl.n_vtiles;
   pl.tiles_per_range = (int)cdiv(pl.n_vtiles, nvr);
@@ -415,7 +417,10 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
     pl.fnP = round_up(n, 8);
     pl.fldL = ncol * pl.fnP;
     pl.fnchunks = cdiv(pl.N, n);
-    const int64_t ntt = cdiv(n, (pl.f_tl || pl.f_sring) ? 256 : 128);
+    // tokens per scan tile (fp32: a separate teacher's logits are staged in L,
+    // in fp32, as the 16-bit ring's are)
+    pl.f_tok = (pl.f_tl || pl.f_sring) ? 256 : (f32 && pl.tsrc == TSRC_SHARED) ? 64 : 128;
+    const int64_t ntt = cdiv(n, pl.f_tok);
     // vocabulary ranges per token tile: the scan's ntt x nvr workgroups stay
     // within scan_groups, so they run in one wave of one per CU (rounding up
     // put 10 token tiles at 260 workgroups, the last 4 a second wave that
@@ -427,12 +432,22 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
     pl.f_nvr = (int)cdiv(pl.n_vtiles, pl.f_tpr);
     // the table's split count is measured for the student's hidden size (the
     // tied teacher's too); a separate teacher's own grad hidden takes the rule
-    auto split_plan = [&](int64_t cols, int& splits, int64_t& kps) -> int {
+    auto split_plan = [&](int64_t cols, bool fine, int& splits, int64_t& kps) -> int {
       int64_t sp = 1;
       if (p->grad_hidden_splits > 0) {
         sp = p->grad_hidden_splits;
       } else if (te && cols == pl.H) {
         sp = te->splits_h;
+      } else if (f32 && fine) {
+        // the least s3_cost over both tile sizes, splits of at least 256 rows
+        double best = 1e30;
+        for (int c = 1; c <= 64 && (c == 1 || pl.V / c >= 256); ++c) {
+          const double cost = std::min(s3_cost(n, cols, pl.V, c, true), s3_cost(n, cols, pl.V, c, false));
+          if (cost < best) {
+            best = cost;
+            sp = c;
+          }
+        }
       } else {
         // Rule: the persistent GEMM runs its tiles x splits equal work items
         // in rounds of kPersistentGroups workgroups, so its time goes as
@@ -466,38 +481,11 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
       splits = (int)cdiv(pl.V, kps);
       return ORDA_OK;
     };
-    ORDA_TRY_PLAN(split_plan(pl.H, pl.splits_s, pl.kps_s));
-    ORDA_TRY_PLAN(split_plan(pl.Ht, pl.splits_t, pl.kps_t));
-    size_t fo = 0;
-    pl.off_L = carve(fo, (size_t)pl.V * pl.fldL * pl.eb);
-    pl.off_fpart = carve(fo, (size_t)pl.f_nvr * kNStat * pl.fnP * 4);
-    pl.off_flabelx = carve(fo, (size_t)2 * pl.fnP * 4);
-    pl.off_frowp = carve(fo, (size_t)kNRowP * pl.fnP * 4);
-    pl.off_frowv = carve(fo, (size_t)3 * pl.N * 4);
-    int64_t split_cols = 0;
-    if ((pl.need_gs || pl.need_gnw) && pl.splits_s > 1) split_cols = pl.splits_s * pl.H;
-    if (pl.w_dln_t && pl.splits_t > 1 && pl.splits_t * pl.Ht > split_cols) split_cols = pl.splits_t * pl.Ht;
-    pl.off_split = split_cols ? carve(fo, (size_t)split_cols * pl.fnP * 4) : 0;
-    // the chunk's hidden states transposed (token-contiguous) for the grad-W
-    // GEMMs: K-major B runs faster on the ring engine than reading them in
-    // place as an MN-major B (measured at C2: 16.4 vs 17.5 ms per step, against
-    // 0.3 ms of transposes)
-    pl.fldh = (tied && pl.w_dlt_t) ? 2 * pl.fnP : pl.fnP;
-    pl.off_fhT = pl.need_gw ? carve(fo, (size_t)pl.H * pl.fldh * pl.eb) : 0;
-    pl.off_fhtT = (sep && pl.need_gwt && pl.w_dlt_t) ? carve(fo, (size_t)pl.Ht * pl.fnP * pl.eb) : 0;
-    pl.off_corr = pl.topk ? carve(fo, (size_t)pl.fnP * p->topk * 4) : 0;
-    pl.off_lse = pl.topk ? carve(fo, (size_t)pl.fnP * 4) : 0;
-    // RMSNorm prologue: the chunk's normalised rows, their rsqrt, dloss/dy when
-    // dloss/dx is not asked for, and the norm weight's gradient sums
-    pl.need_dy = pl.need_gs || pl.need_gnw;
-    pl.norm_groups = (int)std::min<int64_t>(128, cdiv(pl.fn, 8));
-    pl.off_hn = pl.norm ? carve(fo, (size_t)pl.fnP * pl.H * pl.eb) : 0;
-    pl.off_rstd = pl.norm ? carve(fo, (size_t)pl.fnP * 4) : 0;
-    pl.off_dy = (pl.need_gnw && !pl.need_gs) ? carve(fo, (size_t)pl.fnP * pl.H * pl.eb) : 0;
-    pl.off_gpart = pl.need_gnw ? carve(fo, (size_t)pl.norm_groups * pl.H * 4) : 0;
-    pl.off_gacc = pl.need_gnw ? carve(fo, (size_t)pl.H * 4) : 0;
-    // fp8 logits: W (V x H bytes + V scale bytes) once per call, the chunk's
-    // student (and tied teacher) rows per chunk
+    auto both_splits = [&](bool fine) -> int {
+      ORDA_TRY_PLAN(split_plan(pl.H, fine, pl.splits_s, pl.kps_s));
+      return split_plan(pl.Ht, fine, pl.splits_t, pl.kps_t);
+    };
+    ORDA_TRY_PLAN(both_splits(true));
     pl.f8 = (p->flags & ORDA_FP8_LOGITS) != 0;
     if (pl.f8) {
       if (pl.eb != 2) return fail(ORDA_EUNSUPPORTED, "ORDA_FP8_LOGITS needs a 16-bit compute dtype");
@@ -509,13 +497,60 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
       if (!ring)
         return fail(ORDA_EUNSUPPORTED, "ORDA_FP8_LOGITS supports a tied teacher, precomputed logits read in place "
                     "(not the power-family divergences) or no teacher term");
-      const int64_t nb = pl.tsrc == TSRC_SHARED ? 2 : 1;
-      pl.off_w8 = carve(fo, (size_t)pl.V * pl.H);
-      pl.off_ew = carve(fo, (size_t)pl.V);
-      pl.off_b8 = carve(fo, (size_t)nb * pl.fnP * pl.H);
-      pl.off_eb = carve(fo, (size_t)nb * pl.fnP);
     }
-    pl.fwd_bytes = fo + kAlign;
+    auto layout = [&]() {
+      size_t fo = 0;
+      pl.off_L = carve(fo, (size_t)pl.V * pl.fldL * pl.eb);
+      pl.off_fpart = carve(fo, (size_t)pl.f_nvr * kNStat * pl.fnP * 4);
+      pl.off_flabelx = carve(fo, (size_t)2 * pl.fnP * 4);
+      pl.off_frowp = carve(fo, (size_t)kNRowP * pl.fnP * 4);
+      pl.off_frowv = carve(fo, (size_t)3 * pl.N * 4);
+      int64_t split_cols = 0;
+      if ((pl.need_gs || pl.need_gnw) && pl.splits_s > 1) split_cols = pl.splits_s * pl.H;
+      if (pl.w_dln_t && pl.splits_t > 1 && pl.splits_t * pl.Ht > split_cols) split_cols = pl.splits_t * pl.Ht;
+      pl.off_split = split_cols ? carve(fo, (size_t)split_cols * pl.fnP * 4) : 0;
+      // the chunk's hidden states transposed (token-contiguous) for the grad-W
+      // GEMMs: K-major B runs faster on the ring engine than reading them in
+      // place as an MN-major B (measured at C2: 16.4 vs 17.5 ms per step, against
+      // 0.3 ms of transposes); fp32 reads them in place
+      pl.fldh = (tied && pl.w_dlt_t) ? 2 * pl.fnP : pl.fnP;
+      pl.off_fhT = (pl.need_gw && !f32) ? carve(fo, (size_t)pl.H * pl.fldh * pl.eb) : 0;
+      pl.off_fhtT = (sep && pl.need_gwt && pl.w_dlt_t && !f32) ? carve(fo, (size_t)pl.Ht * pl.fnP * pl.eb) : 0;
+      pl.off_corr = pl.topk ? carve(fo, (size_t)pl.fnP * p->topk * 4) : 0;
+      pl.off_lse = pl.topk ? carve(fo, (size_t)pl.fnP * 4) : 0;
+      // RMSNorm prologue: the chunk's normalised rows, their rsqrt, dloss/dy when
+      // dloss/dx is not asked for, and the norm weight's gradient sums
+      pl.need_dy = pl.need_gs || pl.need_gnw;
+      pl.norm_groups = (int)std::min<int64_t>(128, cdiv(pl.fn, 8));
+      pl.off_hn = pl.norm ? carve(fo, (size_t)pl.fnP * pl.H * pl.eb) : 0;
+      pl.off_rstd = pl.norm ? carve(fo, (size_t)pl.fnP * 4) : 0;
+      pl.off_dy = (pl.need_gnw && !pl.need_gs) ? carve(fo, (size_t)pl.fnP * pl.H * pl.eb) : 0;
+      pl.off_gpart = pl.need_gnw ? carve(fo, (size_t)pl.norm_groups * pl.H * 4) : 0;
+      pl.off_gacc = pl.need_gnw ? carve(fo, (size_t)pl.H * 4) : 0;
+      // fp8 logits: W (V x H bytes + V scale bytes) once per call, the chunk's
+      // student (and tied teacher) rows per chunk
+      if (pl.f8) {
+        const int64_t nb = pl.tsrc == TSRC_SHARED ? 2 : 1;
+        pl.off_w8 = carve(fo, (size_t)pl.V * pl.H);
+        pl.off_ew = carve(fo, (size_t)pl.V);
+        pl.off_b8 = carve(fo, (size_t)nb * pl.fnP * pl.H);
+        pl.off_eb = carve(fo, (size_t)nb * pl.fnP);
+      }
+      pl.fwd_bytes = fo + kAlign;
+    };
+    layout();
+    if (f32 && pl.fwd_bytes > ORDA_STATIC_SCRATCH_BYTES) {
+      // a call that the static entry takes keeps fitting: the vocabulary
+      // ranges of 128-token tiles and at most 16 splits, where the finer ones
+      // pass its scratch and those do not
+      const Plan fine = pl;
+      const int64_t coarse = std::min<int64_t>(std::max<int64_t>(kPersistentGroups / cdiv(n, 128), 1), pl.f_nvr);
+      pl.f_tpr = (int)cdiv(pl.n_vtiles, coarse);
+      pl.f_nvr = (int)cdiv(pl.n_vtiles, pl.f_tpr);
+      ORDA_TRY_PLAN(both_splits(false));
+      layout();
+      if (pl.fwd_bytes > ORDA_STATIC_SCRATCH_BYTES) pl = fine;
+    }
     pl.bwd_bytes = 0;
   }
   return ORDA_OK;
@@ -732,7 +767,8 @@ int run_backward(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* 
   F.temperature = p->temperature; F.invT = 1.0f / p->temperature;
   F.alpha = p->div_alpha; F.beta = p->div_beta;
   set_mix(F.mix_w, F.mix_w1, p);
-  F.n_ttiles = pl.n_ttiles; F.rowp = rowp;
+  const int n_ttiles = (int)cdiv(N, 128);  // k_dl's
+  F.n_ttiles = n_ttiles; F.rowp = rowp;
   F.w_s = p->student_ce_weight; F.w_t = p->teacher_ce_weight; F.w_kl = pl.div_on ? p->kl_weight : 0.f;
   // fp16: unscaled dlogits (scal[2] = 1); the gradients get grad_output x
   // mean_scale at the end
@@ -761,7 +797,7 @@ int run_backward(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* 
       if (pl.w_dln_t) { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(dLNt, pl.Vc, N, vcc, vck, eb, s)); }
     }
     F.vc0 = vc0; F.vcc = vcc;
-    const int grid = (int)(cdiv(vcc, 256) * pl.n_ttiles);
+    const int grid = (int)(cdiv(vcc, 256) * n_ttiles);
     {
       const double kt = (pl.bwd_tsrc == TSRC_SHARED || pl.bwd_tsrc == TSRC_SEP) ? (double)Ht : 0.0;
       Timed tm_(ORDA_K_DLOGITS, s, 0.0, 2.0 * (double)N * (double)vcc * ((double)H + kt));
@@ -817,6 +853,21 @@ int gemm2(int la, int lb, const void* A, int64_t lda, const void* B, int64_t ldb
   if ((int64_t)G.tiles_m * G.tiles_n * G.splits > 0x7fffffffll) return fail(ORDA_EINVAL, "gemm grid too large");
   Timed tm_(kind, s, alg, 2.0 * (double)M * (double)N * (double)K);
   ORDA_CHECK_LAUNCH(launch_gemm2<T>(G, s));
+  return ORDA_OK;
+}
+
+// fp32 GEMM on the split-operand engine (launch_gemm_s3); an MN-major B has its
+// K rows [0, seg) from B (val0 valid) and the rest from B1 (val1 valid) when B1.
+inline int gemm_s3(int la, int lb, const void* A, int64_t lda, const void* B, const void* B1, int64_t ldb, int64_t seg,
+                   int64_t val0, int64_t val1, void* C, float* C32, int64_t ldc, int64_t M, int64_t N, int64_t K,
+                   int mode, int splits, int64_t kps, hipStream_t s, int kind, double alg) {
+  GemmParams G{};
+  G.A = A; G.B = B; G.B1 = B1; G.C = C; G.C32 = C32;
+  G.M = M; G.N = N; G.K = K; G.lda = lda; G.ldb = ldb; G.ldb1 = ldb; G.ldc = ldc;
+  G.la = la; G.lb = lb; G.mode = mode; G.b_kseg = seg; G.b_kval0 = val0; G.b_kval1 = val1;
+  G.splits = splits; G.k_per_split = splits > 1 ? kps : K; G.split_stride = M * ldc;
+  Timed tm_(kind, s, alg, 2.0 * (double)M * (double)N * (double)K);
+  ORDA_CHECK_LAUNCH(launch_gemm_s3(G, s));
   return ORDA_OK;
 }
 
@@ -937,13 +988,12 @@ int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, 
     set_mix(F.mix_w, F.mix_w1, p);
     for (int i = 0; i < 3; ++i) { F.pa[i] = pl.pa[i]; F.pb[i] = pl.pb[i]; }
     F.npow = pl.npow;
-    F.phase = 0; F.n_ttiles = (int)cdiv(nc, 128); F.n_vranges = pl.f_nvr;
+    F.phase = 0; F.n_ttiles = (int)cdiv(nc, pl.f_tok); F.n_vranges = pl.f_nvr;
     F.tiles_per_range = pl.f_tpr; F.n_vtiles = pl.n_vtiles;
     F.partial = part; F.rowp = rowp;
     F.Lout = L; F.ldL = ldL; F.tcolL = nP; F.store_t = pl.store_t;
     F.student_ring = pl.f_sring ? 1 : 0;
     F.W8 = w8; F.hs8 = hs8; F.ht8 = ht8; F.eW = ew; F.eS = es; F.eT = et;
-    if (pl.f_sring) F.n_ttiles = (int)cdiv(nc, 256);
     // teacher logits from memory are no GEMM
     bool tgemm = pl.tsrc == TSRC_SHARED || pl.tsrc == TSRC_SEP;
     if (pl.f_tl) {
@@ -970,8 +1020,15 @@ int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, 
                           GEMM_STORE, 1, 0, s, ORDA_K_SCAN, 2.0 * (double)nc * (double)V * (double)Ht));
       }
       if (F.tsrc != TSRC_MEM_RING) F.tsrc = TSRC_L;
-      F.n_ttiles = (int)cdiv(nc, 256);
       tgemm = false;
+    }
+    if constexpr (sizeof(T) == 4) {
+      if (pl.tsrc == TSRC_SEP) {
+        ORDA_TRY(gemm_s3(KMAJ, KMAJ, Wt, Ht, ht + r0 * Ht, nullptr, Ht, 0, 0, 0, L + nP * eb, nullptr, ldL, V, nc, Ht,
+                         GEMM_STORE, 1, 0, s, ORDA_K_SCAN, 2.0 * (double)nc * (double)V * (double)Ht));
+        F.tsrc = TSRC_L;
+        tgemm = false;
+      }
     }
     const double scan_flops = 2.0 * (double)nc * (double)V * ((double)H + (tgemm ? (double)Ht : 0.0));
     if (pl.f8) {
@@ -1049,8 +1106,9 @@ int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, 
     { Timed tm_(ORDA_K_DLOGITS, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_dlm<T>(D, s)); }
     if (pl.topk && pl.div_on) { Timed tm_(ORDA_K_DLOGITS, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_topk_scatter<T>(K, s)); }
 
-    // grad W (+)= dL^T [hs; ht] with both operands K-major over tokens: the
-    // chunk's hidden states are transposed into hT (padding columns zero)
+    // grad W (+)= dL^T [hs; ht]: 16-bit with both operands K-major over tokens
+    // (the chunk's hidden states transposed into hT, padding columns zero),
+    // fp32 with the hidden states read where they are
     const int wmode = c == 0 ? GEMM_STORE : GEMM_ACC_T;
     auto transpose_chunk = [&](const T* src, int64_t cols, char* dst, int64_t ldd, int64_t col0) -> int {
       { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(src, cols, dst + col0 * eb, ldd, nc, nP, cols, s)); }
@@ -1058,28 +1116,45 @@ int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, 
     };
     if (pl.need_gw) {
       const bool both = tied && pl.w_dlt_t;
-      char* hT = ws + pl.off_fhT;
-      ORDA_TRY(transpose_chunk(hsc, H, hT, pl.fldh, 0));
-      if (both) ORDA_TRY(transpose_chunk(ht + r0 * H, H, hT, pl.fldh, nP));
       const int64_t K = both ? 2 * nP : nP;
-      ORDA_TRY(gemm2<T>(KMAJ, KMAJ, L, ldL, hT, pl.fldh, nullptr, 0, K, K, 0, t->grad_weight, nullptr, H, V, H, K,
-                        wmode, 1, 0, s, ORDA_K_GEMM_W, 2.0 * (double)V * (double)H * (double)(both ? 2 * nc : nc)));
+      const double fl = 2.0 * (double)V * (double)H * (double)(both ? 2 * nc : nc);
+      if constexpr (sizeof(T) == 4) {
+        ORDA_TRY(gemm_s3(KMAJ, MNMAJ, L, ldL, hsc, both ? ht + r0 * H : nullptr, H, nP, nc, nc, t->grad_weight, nullptr, H,
+                         V, H, K, wmode, 1, 0, s, ORDA_K_GEMM_W, fl));
+      } else {
+        char* hT = ws + pl.off_fhT;
+        ORDA_TRY(transpose_chunk(hsc, H, hT, pl.fldh, 0));
+        if (both) ORDA_TRY(transpose_chunk(ht + r0 * H, H, hT, pl.fldh, nP));
+        ORDA_TRY(gemm2<T>(KMAJ, KMAJ, L, ldL, hT, pl.fldh, nullptr, 0, K, K, 0, t->grad_weight, nullptr, H, V, H, K,
+                          wmode, 1, 0, s, ORDA_K_GEMM_W, fl));
+      }
     }
     if (sep && pl.need_gwt && pl.w_dlt_t) {
-      char* htT = ws + pl.off_fhtT;
-      ORDA_TRY(transpose_chunk(ht + r0 * Ht, Ht, htT, nP, 0));
-      ORDA_TRY(gemm2<T>(KMAJ, KMAJ, static_cast<char*>(L) + nP * eb, ldL, htT, nP, nullptr, 0, nP, nP, 0,
-                        t->grad_teacher_weight, nullptr, Ht, V, Ht, nP, wmode, 1, 0, s, ORDA_K_GEMM_W,
-                        2.0 * (double)V * (double)Ht * (double)nc));
+      const double fl = 2.0 * (double)V * (double)Ht * (double)nc;
+      const char* Lt = static_cast<char*>(L) + nP * eb;
+      if constexpr (sizeof(T) == 4) {
+        ORDA_TRY(gemm_s3(KMAJ, MNMAJ, Lt, ldL, ht + r0 * Ht, nullptr, Ht, nP, nc, 0, t->grad_teacher_weight, nullptr, Ht, V,
+                         Ht, nP, wmode, 1, 0, s, ORDA_K_GEMM_W, fl));
+      } else {
+        char* htT = ws + pl.off_fhtT;
+        ORDA_TRY(transpose_chunk(ht + r0 * Ht, Ht, htT, nP, 0));
+        ORDA_TRY(gemm2<T>(KMAJ, KMAJ, Lt, ldL, htT, nP, nullptr, 0, nP, nP, 0, t->grad_teacher_weight, nullptr, Ht, V,
+                          Ht, nP, wmode, 1, 0, s, ORDA_K_GEMM_W, fl));
+      }
     }
     // (dst: the chunk's first output row)
     auto grad_hidden = [&](const char* Lcol, const T* Wx, int64_t Hx, T* dst, int splits, int64_t kps) -> int {
       const double fl = 2.0 * (double)nc * (double)Hx * (double)V;
-      if (splits <= 1)
-        return gemm2<T>(MNMAJ, MNMAJ, Lcol, ldL, Wx, Hx, nullptr, 0, V, V, 0, dst, nullptr, Hx, nc, Hx, V,
-                        GEMM_STORE, 1, 0, s, ORDA_K_GEMM_H, fl);
-      ORDA_TRY(gemm2<T>(MNMAJ, MNMAJ, Lcol, ldL, Wx, Hx, nullptr, 0, V, V, 0, nullptr, split, Hx, nc, Hx, V,
-                        GEMM_SPLIT, splits, kps, s, ORDA_K_GEMM_H, fl));
+      const int mode = splits <= 1 ? GEMM_STORE : GEMM_SPLIT;
+      void* C = splits <= 1 ? dst : nullptr;
+      float* C32 = splits <= 1 ? nullptr : split;
+      if constexpr (sizeof(T) == 4)
+        ORDA_TRY(gemm_s3(MNMAJ, MNMAJ, Lcol, ldL, Wx, nullptr, Hx, 0, V, 0, C, C32, Hx, nc, Hx, V, mode, splits, kps, s,
+                         ORDA_K_GEMM_H, fl));
+      else
+        ORDA_TRY(gemm2<T>(MNMAJ, MNMAJ, Lcol, ldL, Wx, Hx, nullptr, 0, V, V, 0, C, C32, Hx, nc, Hx, V, mode, splits,
+                          kps, s, ORDA_K_GEMM_H, fl));
+      if (splits <= 1) return ORDA_OK;
       Timed tm_(ORDA_K_AUX, s, 0.0, 0.0);
       ORDA_CHECK_LAUNCH(launch_splitk_reduce<T>(split, splits, nc * Hx, dst, Hx, nc, Hx, s));
       return ORDA_OK;

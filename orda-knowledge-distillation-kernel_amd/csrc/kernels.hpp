@@ -164,6 +164,13 @@ struct AccPair4 {  // ring engine, the lane's token j: acc[mb][j] student, acc[m
 template <class AP>
 __device__ __forceinline__ void acc_fence(const AP&) {}
 
+// Accessors whose lane may hold teacher logits that are all -inf (a masked
+// stretch of the vocabulary) in one tile: 16 rows per lane instead of 64 or
+// 32.  The maxima they rescale by are then taken as 0 (exp(-inf) adds
+// nothing) instead of forming -inf - -inf.
+template <class AP>
+struct GuardMasked : std::false_type {};
+
 // Phase 0: online softmax statistics of this lane's token over its
 // vocabulary rows of the tile (64 or 32, AP::Lay).  Template flags remove work that the problem
 // does not need (NPOW: the power family's terms, 1 or up to 3, P.npow).
@@ -206,7 +213,8 @@ __device__ __forceinline__ void scan_tile(RowState& S, const AP& acc, int vlane0
   float nmt = 0.f;
   if (HAS_T) {
     nmt = fmaxf(S.mt, tmt);
-    const float d = S.mt - nmt;
+    const bool none = GuardMasked<AP>::value && nmt == -kInf;  // every teacher logit so far is -inf
+    const float d = none ? 0.f : S.mt - nmt;
     const float ct = fexp(d);
     const float ctT = T1 ? ct : fexp(d * invT);
     if (FAM == FAM_LIN) {
@@ -217,22 +225,20 @@ __device__ __forceinline__ void scan_tile(RowState& S, const AP& acc, int vlane0
     S.st *= ct;
     if (!T1) S.stt *= ctT;
     S.mt = nmt;
+    if (none) nmt = 0.f;
   }
   float nmu0 = 0.f, nmu1 = 0.f, nmu2 = 0.f;
   if (FAM == FAM_POW) {
-    nmu0 = fmaxf(S.x[0], tmu0 * invT);
-    S.x[1] *= fexp(S.x[0] - nmu0);
-    S.x[0] = nmu0;
-    if (NPOW > 1 && P.npow > 1) {
-      nmu1 = fmaxf(S.x[2], tmu1 * invT);
-      S.x[3] *= fexp(S.x[2] - nmu1);
-      S.x[2] = nmu1;
-    }
-    if (NPOW > 2 && P.npow > 2) {
-      nmu2 = fmaxf(S.x[4], tmu2 * invT);
-      S.x[5] *= fexp(S.x[4] - nmu2);
-      S.x[4] = nmu2;
-    }
+    auto to_max = [&](float& m, float& sum, float tile_max) __attribute__((always_inline)) {
+      const float nm = fmaxf(m, tile_max);
+      const bool none = GuardMasked<AP>::value && nm == -kInf;
+      sum *= none ? 1.f : fexp(m - nm);
+      m = nm;
+      return none ? 0.f : nm;
+    };
+    nmu0 = to_max(S.x[0], S.x[1], tmu0 * invT);
+    if (NPOW > 1 && P.npow > 1) nmu1 = to_max(S.x[2], S.x[3], tmu1 * invT);
+    if (NPOW > 2 && P.npow > 2) nmu2 = to_max(S.x[4], S.x[5], tmu2 * invT);
   }
 
   // accumulate this tile.  exp(x - m) = 2^(x log2e - m log2e): one fma forms

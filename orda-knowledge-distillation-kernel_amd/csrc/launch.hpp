@@ -210,6 +210,24 @@ template <class T> hipError_t launch_scan_store(const FusedParams& P, int grid, 
 template <class T> hipError_t launch_scan_store_f8(const FusedParams& P, int grid, hipStream_t s);
 template <class T> hipError_t launch_quant_f8(const QuantParams& P, hipStream_t s);
 template <class T> hipError_t launch_gemm2(const GemmParams& P, hipStream_t s);
+// fp32: la, lb and mode as k_gemm_s3 has them (tiles by s3_cost)
+hipError_t launch_gemm_s3(GemmParams P, hipStream_t s);
+
+// Estimated microseconds of an M x N x K fp32 GEMM in `splits` K ranges on
+// large (256 x 128, one workgroup to a CU) or small (64 x 64, three) tiles:
+// rounds of resident workgroups times the K steps of one, plus a round's
+// start and write-out, plus the partials' way out and back.  Measured: 2.7 us
+// per 32-deep step of a large tile (30001 x 1000 x 1000: 349 us, 4 rounds of 32
+// steps) and 1.1-1.5 of a small one (512 x 256 x 4096 in 16 splits: 16.6 us;
+// 320 x 584 x 29568 in 16: 188 us, 2 rounds of 58).
+inline double s3_cost(double M, double N, double K, int splits, bool large) {
+  auto up = [](double a, double b) { const double q = a / b; return (double)(int64_t)(q + 0.999999); };
+  const double items = (large ? up(M, 256) * up(N, 128) : up(M, 64) * up(N, 64)) * splits;
+  const double steps = up(K / splits, 32);
+  const double rounds = up(items, large ? 256 : 768);
+  const double part = splits > 1 ? splits * M * N * 8.0 / 4e6 : 0.0;
+  return rounds * (large ? steps * 2.7 + 8.0 : steps * 1.5 + 7.0) + part;
+}
 template <class T> hipError_t launch_dlm(const DlmParams& P, hipStream_t s);
 template <class T> hipError_t launch_topk_rows(const TopKParams& P, hipStream_t s);
 template <class T> hipError_t launch_topk_scatter(const TopKParams& P, hipStream_t s);
