@@ -706,17 +706,20 @@ int gemm(const void* A, int64_t lda, const void* B, int64_t ldb, void* C, float*
 // returns at once when it is 1).
 template <class T>
 int scale_grads(const Plan& pl, const orda_tensors_t* t, const float* factor, hipStream_t s) {
-  auto sc = [&](void* g, int64_t n) -> int {
-    if (!g) return ORDA_OK;
-    Timed tm_(ORDA_K_AUX, s, 0.0, 0.0);
-    ORDA_CHECK_LAUNCH(launch_scale<T>(g, n, factor, s));
-    return ORDA_OK;
+  ScaleParams S{};
+  S.g = factor;
+  auto add = [&](void* g, int64_t n) {
+    if (!g) return;
+    S.x[S.count] = g;
+    S.n[S.count++] = n;
   };
-  if (pl.need_gs) ORDA_TRY(sc(t->grad_student_hidden, pl.N * pl.H));
-  if (pl.need_gw) ORDA_TRY(sc(t->grad_weight, pl.V * pl.H));
-  if (pl.need_gt) ORDA_TRY(sc(t->grad_teacher_hidden, pl.N * pl.Ht));
-  if (pl.need_gwt) ORDA_TRY(sc(t->grad_teacher_weight, pl.V * pl.Ht));
-  if (pl.need_gnw) ORDA_TRY(sc(t->grad_student_norm_weight, pl.H));
+  if (pl.need_gs) add(t->grad_student_hidden, pl.N * pl.H);
+  if (pl.need_gw) add(t->grad_weight, pl.V * pl.H);
+  if (pl.need_gt) add(t->grad_teacher_hidden, pl.N * pl.Ht);
+  if (pl.need_gwt) add(t->grad_teacher_weight, pl.V * pl.Ht);
+  if (pl.need_gnw) add(t->grad_student_norm_weight, pl.H);
+  Timed tm_(ORDA_K_AUX, s, 0.0, 0.0);
+  ORDA_CHECK_LAUNCH(launch_scale<T>(S, s));
   return ORDA_OK;
 }
 
@@ -748,9 +751,10 @@ int run_backward(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* 
   // Transposed hidden states for the grad_W GEMMs (K = tokens), with zeroed
   // padding columns so K can be rounded up to a multiple of 8.
   if (pl.need_gw) {
-    { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(t->student_hidden, H, hT, pl.ldh, N, NP, H, s)); }
-    if (tied && pl.w_dlt_t)
-      { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(t->teacher_hidden, H, hT + NP * eb, pl.ldh, N, NP, H, s)); }
+    const bool both = tied && pl.w_dlt_t;
+    Timed tm_(ORDA_K_AUX, s, 0.0, 0.0);
+    ORDA_CHECK_LAUNCH(launch_transpose<T>(t->student_hidden, H, hT, pl.ldh, N, NP, H, s,
+                                          both ? t->teacher_hidden : nullptr, both ? hT + NP * eb : nullptr));
   }
   if (sep && pl.w_dlt_t)
     { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(t->teacher_hidden, Ht, htT, NP, N, NP, Ht, s)); }
@@ -922,9 +926,6 @@ int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, 
     Timed tm_(ORDA_K_AUX, s, 0.0, 0.0);
     ORDA_CHECK_LAUNCH(launch_quant_f8<T>(Q, s));
   }
-  // mean scale first: the chunks' dlogits need it before the loss rows exist
-  { Timed tm_(ORDA_K_ROWS, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_count(t->labels, N, p->ignore_index, reduction_sum, scal, s)); }
-
   for (int64_t c = 0; c < pl.fnchunks; ++c) {
     const int64_t r0 = c * pl.fn;
     const int64_t nc = (N - r0 < pl.fn) ? N - r0 : pl.fn;
@@ -974,6 +975,9 @@ int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, 
     Lb.N = nc; Lb.V = V; Lb.H = H; Lb.Ht = Ht; Lb.ignore_index = p->ignore_index;
     Lb.tsrc = pl.tsrc; Lb.lt_dtype = p->logits_dtype; Lb.out = labelx;
     Lb.W8 = w8; Lb.hs8 = hs8; Lb.ht8 = ht8; Lb.eW = ew; Lb.eS = es; Lb.eT = et;
+    if (c == 0) {  // and the mean scale of the whole call, which the chunks' dlogits need
+      Lb.scal = scal; Lb.all_labels = t->labels; Lb.all_N = N; Lb.reduction_sum = reduction_sum;
+    }
     { Timed tm_(ORDA_K_ROWS, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_label<T>(Lb, s)); }
 
     FusedParams F{};
@@ -1110,8 +1114,9 @@ int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, 
     // (the chunk's hidden states transposed into hT, padding columns zero),
     // fp32 with the hidden states read where they are
     const int wmode = c == 0 ? GEMM_STORE : GEMM_ACC_T;
-    auto transpose_chunk = [&](const T* src, int64_t cols, char* dst, int64_t ldd, int64_t col0) -> int {
-      { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(src, cols, dst + col0 * eb, ldd, nc, nP, cols, s)); }
+    auto transpose_chunk = [&](const T* src, const T* src1, int64_t cols, char* dst, int64_t ldd) -> int {
+      Timed tm_(ORDA_K_AUX, s, 0.0, 0.0);
+      ORDA_CHECK_LAUNCH(launch_transpose<T>(src, cols, dst, ldd, nc, nP, cols, s, src1, src1 ? dst + nP * eb : nullptr));
       return ORDA_OK;
     };
     if (pl.need_gw) {
@@ -1123,8 +1128,7 @@ int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, 
                          V, H, K, wmode, 1, 0, s, ORDA_K_GEMM_W, fl));
       } else {
         char* hT = ws + pl.off_fhT;
-        ORDA_TRY(transpose_chunk(hsc, H, hT, pl.fldh, 0));
-        if (both) ORDA_TRY(transpose_chunk(ht + r0 * H, H, hT, pl.fldh, nP));
+        ORDA_TRY(transpose_chunk(hsc, both ? ht + r0 * H : nullptr, H, hT, pl.fldh));
         ORDA_TRY(gemm2<T>(KMAJ, KMAJ, L, ldL, hT, pl.fldh, nullptr, 0, K, K, 0, t->grad_weight, nullptr, H, V, H, K,
                           wmode, 1, 0, s, ORDA_K_GEMM_W, fl));
       }
@@ -1137,7 +1141,7 @@ int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, 
                          Ht, nP, wmode, 1, 0, s, ORDA_K_GEMM_W, fl));
       } else {
         char* htT = ws + pl.off_fhtT;
-        ORDA_TRY(transpose_chunk(ht + r0 * Ht, Ht, htT, nP, 0));
+        ORDA_TRY(transpose_chunk(ht + r0 * Ht, nullptr, Ht, htT, nP));
         ORDA_TRY(gemm2<T>(KMAJ, KMAJ, Lt, ldL, htT, nP, nullptr, 0, nP, nP, 0, t->grad_teacher_weight, nullptr, Ht, V,
                           Ht, nP, wmode, 1, 0, s, ORDA_K_GEMM_W, fl));
       }
@@ -1418,10 +1422,12 @@ int orda_scale_gradient(int32_t dtype, void* grad, int64_t numel, const float* f
   if (!aligned16(grad)) return fail(ORDA_EINVAL, "grad must be 16-byte aligned");
   hipStream_t s = static_cast<hipStream_t>(stream);
   Timed tm_(ORDA_K_AUX, s, 0.0, 0.0);
+  ScaleParams S{};
+  S.x[0] = grad; S.n[0] = numel; S.count = 1; S.g = factor;
   switch (dtype) {
-    case ORDA_BF16: ORDA_CHECK_LAUNCH(launch_scale<bf16>(grad, numel, factor, s)); break;
-    case ORDA_F16: ORDA_CHECK_LAUNCH(launch_scale<f16>(grad, numel, factor, s)); break;
-    case ORDA_F32: ORDA_CHECK_LAUNCH(launch_scale<float>(grad, numel, factor, s)); break;
+    case ORDA_BF16: ORDA_CHECK_LAUNCH(launch_scale<bf16>(S, s)); break;
+    case ORDA_F16: ORDA_CHECK_LAUNCH(launch_scale<f16>(S, s)); break;
+    case ORDA_F32: ORDA_CHECK_LAUNCH(launch_scale<float>(S, s)); break;
     default: return fail(ORDA_EINVAL, "unknown dtype %d", dtype);
   }
   return ORDA_OK;

@@ -1971,12 +1971,14 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(const float* __restrict__
   store4(out + m * ldo + c, x, true, 4);
 }
 
-// x *= g[0] in place (n elements, n a multiple of 4, x 8-byte aligned);
-// nothing to do when g[0] == 1.
+// x *= g[0] in place for each buffer (blockIdx.y; 16-byte aligned); nothing
+// to do when g[0] == 1, the usual case of a backward from the loss itself.
 template <class T>
-__global__ __launch_bounds__(256) void k_scale(T* __restrict__ x, int64_t n, const float* __restrict__ g) {
-  const float s = g[0];
+__global__ __launch_bounds__(256) void k_scale(ScaleParams P) {
+  const float s = P.g[0];
   if (s == 1.0f) return;
+  T* __restrict__ x = static_cast<T*>(P.x[blockIdx.y]);
+  const int64_t n = P.n[blockIdx.y];
   for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4; i < n; i += (int64_t)gridDim.x * 256 * 4) {
     const int cnt = (int)min<int64_t>(4, n - i);  // (a ragged tail element by element)
     float v[4];
@@ -2462,9 +2464,13 @@ __global__ __launch_bounds__(256) void k_dlm_tm(DlmParams P) {
 // tid / 8 + 32, piece tid % 8 (8 columns) on the way in; output rows the same
 // on the way out, each piece gathered from 8 tile rows.
 template <class T>
-__global__ __launch_bounds__(256) void k_transpose(const T* __restrict__ in, int64_t ldi, T* __restrict__ out,
-                                                   int64_t ldo, int64_t R, int64_t Rp, int64_t C, int tiles_c,
-                                                   int vec) {
+__global__ __launch_bounds__(256) void k_transpose(const T* __restrict__ in, const T* __restrict__ in1, int64_t ldi,
+                                                   T* __restrict__ out, T* __restrict__ out1, int64_t ldo, int64_t R,
+                                                   int64_t Rp, int64_t C, int tiles_c, int vec) {
+  if (blockIdx.y) {  // the second matrix of the launch
+    in = in1;
+    out = out1;
+  }
   __shared__ __align__(16) T tile[64][72];  // (pitch 144 bytes: 16-byte aligned rows)
   const int tr = blockIdx.x / tiles_c, tc = blockIdx.x % tiles_c;
   const int64_t r0 = (int64_t)tr * 64, c0 = (int64_t)tc * 64;
@@ -2646,8 +2652,38 @@ __device__ __forceinline__ float row_dot_f8(const uint8_t* a, const uint8_t* b, 
   return acc;
 }
 
+// The last workgroup's count of non-ignored labels and the mean scale, as
+// k_finalize computes them: the chunks' dlogits need the scale before the
+// loss rows exist.
+__device__ __forceinline__ void count_labels(const LabelParams& P) {
+  __shared__ int64_t part[4];
+  int64_t n = 0;
+  constexpr int U = 8;  // loads in flight
+  for (int64_t t = threadIdx.x; t < P.all_N; t += 256 * U) {
+    int64_t y[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) y[u] = t + 256 * u < P.all_N ? P.all_labels[t + 256 * u] : P.ignore_index;
+#pragma unroll
+    for (int u = 0; u < U; ++u) n += y[u] != P.ignore_index ? 1 : 0;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = n;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  const double count = (double)(part[0] + part[1] + part[2] + part[3]);
+  const double denom = count < 1.0 ? 1.0 : count;
+  P.scal[0] = P.reduction_sum ? 1.0f : 1.0f / (float)denom;
+  P.scal[1] = (float)count;
+  P.scal[2] = 1.0f;
+}
+
 template <class T>
 __global__ __launch_bounds__(256) void k_label(LabelParams P) {
+  if (P.scal && blockIdx.x == gridDim.x - 1) {
+    count_labels(P);
+    return;
+  }
   const int lane = threadIdx.x & 63;
   const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (t >= P.N) return;
@@ -2790,12 +2826,14 @@ hipError_t launch_gemm(const GemmParams& P, hipStream_t s) {
 }
 template <class T>
 hipError_t launch_transpose(const void* in, int64_t ldi, void* out, int64_t ldo, int64_t R, int64_t Rp, int64_t C,
-                            hipStream_t s) {
+                            hipStream_t s, const void* in1, void* out1) {
   const int tiles_r = (int)((Rp + 63) / 64), tiles_c = (int)((C + 63) / 64);
-  const int vec = sizeof(T) == 2 && ldi % 8 == 0 && ldo % 8 == 0 && reinterpret_cast<uintptr_t>(in) % 16 == 0 &&
-                  reinterpret_cast<uintptr_t>(out) % 16 == 0;
-  hipLaunchKernelGGL(k_transpose<T>, dim3(tiles_r * tiles_c), dim3(256), 0, s, static_cast<const T*>(in), ldi,
-                     static_cast<T*>(out), ldo, R, Rp, C, tiles_c, vec);
+  const uintptr_t all = reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out) |
+                        reinterpret_cast<uintptr_t>(in1) | reinterpret_cast<uintptr_t>(out1);
+  const int vec = sizeof(T) == 2 && ldi % 8 == 0 && ldo % 8 == 0 && all % 16 == 0;
+  hipLaunchKernelGGL(k_transpose<T>, dim3(tiles_r * tiles_c, in1 ? 2 : 1), dim3(256), 0, s, static_cast<const T*>(in),
+                     static_cast<const T*>(in1), ldi, static_cast<T*>(out), static_cast<T*>(out1), ldo, R, Rp, C,
+                     tiles_c, vec);
   return hipGetLastError();
 }
 
@@ -2826,7 +2864,7 @@ hipError_t launch_transpose_cast(const void* in, int in_dtype, int64_t ldi, void
 
 template <class T>
 hipError_t launch_label(const LabelParams& P, hipStream_t s) {
-  const int grid = (int)((P.N + 3) / 4);
+  const int grid = (int)((P.N + 3) / 4) + (P.scal ? 1 : 0);
   hipLaunchKernelGGL(k_label<T>, dim3(grid), dim3(256), 0, s, P);
   return hipGetLastError();
 }
@@ -3379,11 +3417,14 @@ inline void dlm_go(const DlmParams& P, hipStream_t s) {
                        stride, static_cast<T*>(out), ldo, M, N);                           \
     return hipGetLastError();                                                              \
   }                                                                                        \
-  template <> hipError_t launch_scale<T>(void* x, int64_t n, const float* g, hipStream_t s) { \
+  template <> hipError_t launch_scale<T>(const ScaleParams& P, hipStream_t s) {            \
+    if (P.count <= 0) return hipSuccess;                                                   \
+    int64_t n = 0;                                                                         \
+    for (int i = 0; i < P.count; ++i) n = P.n[i] > n ? P.n[i] : n;                         \
     int64_t blocks = (n / 4 + 255) / 256;                                                  \
     if (blocks > 8192) blocks = 8192;                                                      \
     if (blocks < 1) blocks = 1;                                                            \
-    hipLaunchKernelGGL(k_scale<T>, dim3((unsigned)blocks), dim3(256), 0, s, static_cast<T*>(x), n, g); \
+    hipLaunchKernelGGL(k_scale<T>, dim3((unsigned)blocks, (unsigned)P.count), dim3(256), 0, s, P); \
     return hipGetLastError();                                                              \
   }
 
@@ -3391,7 +3432,7 @@ inline void dlm_go(const DlmParams& P, hipStream_t s) {
   template hipError_t launch_gemm<T>(const GemmParams&, hipStream_t);                                \
   template hipError_t launch_label<T>(const LabelParams&, hipStream_t);                              \
   template hipError_t launch_transpose<T>(const void*, int64_t, void*, int64_t, int64_t, int64_t, int64_t, \
-                                          hipStream_t);                                              \
+                                          hipStream_t, const void*, void*);                                              \
   template hipError_t launch_transpose_cast<T>(const void*, int, int64_t, void*, int64_t, int64_t, int64_t, \
                                                hipStream_t);
 

@@ -190,6 +190,20 @@ struct LabelParams {
   const uint8_t* eW;
   const uint8_t* eS;
   const uint8_t* eT;
+  // when set, one more workgroup writes the mean scale and count of all_N
+  // labels there (scal[0 .. 2] as k_finalize)
+  float* scal;
+  const int64_t* all_labels;
+  int64_t all_N;
+  int reduction_sum;
+};
+
+// Up to five buffers of T multiplied in place by one device scalar (k_scale).
+struct ScaleParams {
+  void* x[5];
+  int64_t n[5];
+  int count;
+  const float* g;
 };
 
 // Rows [rows x H] (compute dtype, pitch H) to OCP e4m3 bytes q [rows x H]
@@ -238,11 +252,12 @@ template <class T> hipError_t launch_two(const TwoParams& P, hipStream_t s);
 template <class T>
 hipError_t launch_splitk_reduce(const float* part, int splits, int64_t stride, void* out, int64_t ldo, int64_t M,
                                 int64_t N, hipStream_t s);
-template <class T> hipError_t launch_scale(void* x, int64_t n, const float* g, hipStream_t s);
-// out[c * ldo + r] = r < R ? in[r * ldi + c] : 0 for r < Rp, c < C
+template <class T> hipError_t launch_scale(const ScaleParams& P, hipStream_t s);
+// out[c * ldo + r] = r < R ? in[r * ldi + c] : 0 for r < Rp, c < C; with in1,
+// the same from in1 to out1 in the same launch
 template <class T>
 hipError_t launch_transpose(const void* in, int64_t ldi, void* out, int64_t ldo, int64_t R, int64_t Rp, int64_t C,
-                            hipStream_t s);
+                            hipStream_t s, const void* in1 = nullptr, void* out1 = nullptr);
 // The same for logits of dtype in_dtype (DT_*), rounded once to T.
 template <class T>
 hipError_t launch_transpose_cast(const void* in, int in_dtype, int64_t ldi, void* out, int64_t ldo, int64_t R,
@@ -289,12 +304,6 @@ struct FinalizeParams {
   float* scal;  // [0] = mean_scale, [1] = count of non-ignored rows, [2] = 1
 };
 hipError_t launch_finalize(const FinalizeParams& P, hipStream_t s);
-
-// scal[0] = mean scale (1 / max(count, 1), or 1 for sum), scal[1] = count of
-// non-ignored labels, scal[2] = 1: the same values k_finalize writes,
-// available before the loss rows exist.
-hipError_t launch_count(const int64_t* labels, int64_t N, int64_t ignore_index, int reduction_sum, float* scal,
-                        hipStream_t s);
 
 // *out = a[0] * b[0] (device scalars; one thread)
 hipError_t launch_mul_scalars(const float* a, const float* b, float* out, hipStream_t s);

@@ -243,28 +243,6 @@ __global__ __launch_bounds__(1024) void k_finalize(FinalizeParams P) {
   }
 }
 
-// Count of non-ignored labels and the mean scale, as k_finalize computes them.
-__global__ __launch_bounds__(1024) void k_count(const int64_t* labels, int64_t N, int64_t ignore_index,
-                                                int reduction_sum, float* scal) {
-  __shared__ double red[1024];
-  const int tid = threadIdx.x;
-  double cnt = 0.0;
-  for (int64_t t = tid; t < N; t += 1024) cnt += (labels[t] != ignore_index) ? 1.0 : 0.0;
-  red[tid] = cnt;
-  __syncthreads();
-  for (int w = 512; w > 0; w >>= 1) {
-    if (tid < w) red[tid] += red[tid + w];
-    __syncthreads();
-  }
-  if (tid == 0) {
-    const double count = red[0];
-    const double denom = count < 1.0 ? 1.0 : count;
-    scal[0] = reduction_sum ? 1.0f : 1.0f / (float)denom;
-    scal[1] = (float)count;
-    scal[2] = 1.0f;
-  }
-}
-
 __global__ void k_mul_scalars(const float* a, const float* b, float* out) { *out = a[0] * b[0]; }
 
 __global__ void k_zero2d(char* out, int64_t ld_bytes, int64_t R, int64_t c0_bytes, int64_t w_bytes) {
@@ -287,11 +265,6 @@ hipError_t launch_finalize(const FinalizeParams& P, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_count(const int64_t* labels, int64_t N, int64_t ignore_index, int reduction_sum, float* scal,
-                        hipStream_t s) {
-  hipLaunchKernelGGL(k_count, dim3(1), dim3(1024), 0, s, labels, N, ignore_index, reduction_sum, scal);
-  return hipGetLastError();
-}
 hipError_t launch_mul_scalars(const float* a, const float* b, float* out, hipStream_t s) {
   hipLaunchKernelGGL(k_mul_scalars, dim3(1), dim3(1), 0, s, a, b, out);
   return hipGetLastError();
