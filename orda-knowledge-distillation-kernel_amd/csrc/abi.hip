@@ -540,13 +540,15 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
     };
     layout();
     if (f32 && pl.fwd_bytes > ORDA_STATIC_SCRATCH_BYTES) {
-      // a call that the static entry takes keeps fitting: the vocabulary
-      // ranges of 128-token tiles and at most 16 splits, where the finer ones
-      // pass its scratch and those do not
+      // a call that the static entry takes keeps fitting: at most 16 splits
+      // (and, in fp32, the vocabulary ranges of 128-token tiles) where more
+      // would pass its scratch and those do not
       const Plan fine = pl;
-      const int64_t coarse = std::min<int64_t>(std::max<int64_t>(kPersistentGroups / cdiv(n, 128), 1), pl.f_nvr);
-      pl.f_tpr = (int)cdiv(pl.n_vtiles, coarse);
-      pl.f_nvr = (int)cdiv(pl.n_vtiles, pl.f_tpr);
+      if (f32) {
+        const int64_t coarse = std::min<int64_t>(std::max<int64_t>(kPersistentGroups / cdiv(n, 128), 1), pl.f_nvr);
+        pl.f_tpr = (int)cdiv(pl.n_vtiles, coarse);
+        pl.f_nvr = (int)cdiv(pl.n_vtiles, pl.f_tpr);
+      }
       ORDA_TRY_PLAN(both_splits(false));
       layout();
       if (pl.fwd_bytes > ORDA_STATIC_SCRATCH_BYTES) pl = fine;
@@ -845,9 +847,10 @@ int run_backward(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* 
 template <class T>
 int gemm2(int la, int lb, const void* A, int64_t lda, const void* B, int64_t ldb, const void* B1, int64_t ldb1,
           int64_t b_kseg, int64_t b_kval0, int64_t b_kval1, void* C, float* C32, int64_t ldc, int64_t M,
-          int64_t N, int64_t K, int mode, int splits, int64_t kps, hipStream_t s, int kind, double alg) {
+          int64_t N, int64_t K, int mode, int splits, int64_t kps, hipStream_t s, int kind, double alg,
+          const float* cscale = nullptr) {
   GemmParams G{};
-  G.A = A; G.B = B; G.C = C; G.C32 = C32;
+  G.A = A; G.B = B; G.C = C; G.C32 = C32; G.cscale = cscale;
   G.M = M; G.N = N; G.K = K; G.lda = lda; G.ldb = ldb; G.ldc = ldc;
   G.tiles_m = (int)cdiv(M, 256); G.tiles_n = (int)cdiv(N, 256); G.mode = mode;
   G.la = la; G.lb = lb; G.B1 = B1; G.ldb1 = ldb1; G.b_kseg = b_kseg; G.b_kval0 = b_kval0; G.b_kval1 = b_kval1;
@@ -1114,6 +1117,13 @@ int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, 
     // (the chunk's hidden states transposed into hT, padding columns zero),
     // fp32 with the hidden states read where they are
     const int wmode = c == 0 ? GEMM_STORE : GEMM_ACC_T;
+    // fp16 (late_scale): the mean scale goes into the GEMMs' last rounding --
+    // grad W's in the last chunk, each chunk's grad hidden rows in theirs
+    // (scaling the finished buffers took another read and write of each: 230
+    // of 2714 us at 2048 tokens, hidden 1024 / 2048, vocabulary 65536, every
+    // gradient).  The norm's backward takes its rows unscaled.
+    const float* const late = pl.late_scale ? scal : nullptr;
+    const float* const late_w = c + 1 == pl.fnchunks ? late : nullptr;
     auto transpose_chunk = [&](const T* src, const T* src1, int64_t cols, char* dst, int64_t ldd) -> int {
       Timed tm_(ORDA_K_AUX, s, 0.0, 0.0);
       ORDA_CHECK_LAUNCH(launch_transpose<T>(src, cols, dst, ldd, nc, nP, cols, s, src1, src1 ? dst + nP * eb : nullptr));
@@ -1130,7 +1140,7 @@ int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, 
         char* hT = ws + pl.off_fhT;
         ORDA_TRY(transpose_chunk(hsc, both ? ht + r0 * H : nullptr, H, hT, pl.fldh));
         ORDA_TRY(gemm2<T>(KMAJ, KMAJ, L, ldL, hT, pl.fldh, nullptr, 0, K, K, 0, t->grad_weight, nullptr, H, V, H, K,
-                          wmode, 1, 0, s, ORDA_K_GEMM_W, fl));
+                          wmode, 1, 0, s, ORDA_K_GEMM_W, fl, late_w));
       }
     }
     if (sep && pl.need_gwt && pl.w_dlt_t) {
@@ -1143,11 +1153,12 @@ int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, 
         char* htT = ws + pl.off_fhtT;
         ORDA_TRY(transpose_chunk(ht + r0 * Ht, nullptr, Ht, htT, nP));
         ORDA_TRY(gemm2<T>(KMAJ, KMAJ, Lt, ldL, htT, nP, nullptr, 0, nP, nP, 0, t->grad_teacher_weight, nullptr, Ht, V,
-                          Ht, nP, wmode, 1, 0, s, ORDA_K_GEMM_W, fl));
+                          Ht, nP, wmode, 1, 0, s, ORDA_K_GEMM_W, fl, late_w));
       }
     }
     // (dst: the chunk's first output row)
-    auto grad_hidden = [&](const char* Lcol, const T* Wx, int64_t Hx, T* dst, int splits, int64_t kps) -> int {
+    auto grad_hidden = [&](const char* Lcol, const T* Wx, int64_t Hx, T* dst, int splits, int64_t kps,
+                           const float* scale) -> int {
       const double fl = 2.0 * (double)nc * (double)Hx * (double)V;
       const int mode = splits <= 1 ? GEMM_STORE : GEMM_SPLIT;
       void* C = splits <= 1 ? dst : nullptr;
@@ -1157,17 +1168,17 @@ int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, 
                          ORDA_K_GEMM_H, fl));
       else
         ORDA_TRY(gemm2<T>(MNMAJ, MNMAJ, Lcol, ldL, Wx, Hx, nullptr, 0, V, V, 0, C, C32, Hx, nc, Hx, V, mode, splits,
-                          kps, s, ORDA_K_GEMM_H, fl));
+                          kps, s, ORDA_K_GEMM_H, fl, scale));
       if (splits <= 1) return ORDA_OK;
       Timed tm_(ORDA_K_AUX, s, 0.0, 0.0);
-      ORDA_CHECK_LAUNCH(launch_splitk_reduce<T>(split, splits, nc * Hx, dst, Hx, nc, Hx, s));
+      ORDA_CHECK_LAUNCH(launch_splitk_reduce<T>(split, splits, nc * Hx, dst, Hx, nc, Hx, scale, s));
       return ORDA_OK;
     };
     if (pl.need_dy) {
       // dloss/dy of the chunk's rows; with the norm, then dloss/dgamma and
       // dloss/dx (in place)
       T* dy = pl.need_gs ? static_cast<T*>(t->grad_student_hidden) + r0 * H : reinterpret_cast<T*>(ws + pl.off_dy);
-      ORDA_TRY(grad_hidden(L, W, H, dy, pl.splits_s, pl.kps_s));
+      ORDA_TRY(grad_hidden(L, W, H, dy, pl.splits_s, pl.kps_s, pl.norm ? nullptr : late));
       if (pl.norm) {
         Nm.dxy = dy;
         if (pl.need_gnw) {
@@ -1182,7 +1193,7 @@ int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, 
     }
     if (pl.w_dln_t)
       ORDA_TRY(grad_hidden(L + nP * eb, tied ? W : Wt, Ht, static_cast<T*>(t->grad_teacher_hidden) + r0 * Ht,
-                           pl.splits_t, pl.kps_t));
+                           pl.splits_t, pl.kps_t, late));
   }
 
   FinalizeParams Z{};
@@ -1198,9 +1209,15 @@ int run_fused(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, 
     { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(t->grad_teacher_hidden, Ht, N, 0, Ht, eb, s)); }
   if (sep && pl.need_gwt && !pl.w_dlt_t)
     { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(t->grad_teacher_weight, Ht, V, 0, Ht, eb, s)); }
-  // fp16: the chunks' dlogits were unscaled; the mean scale once here (the
-  // backward applies grad_output)
-  if (pl.late_scale && any_grad) ORDA_TRY(scale_grads<T>(pl, t, scal, s));
+  // fp16 behind the norm: its backward ran on unscaled rows
+  if (pl.late_scale && pl.norm && pl.need_dy) {
+    ScaleParams S{};
+    S.g = scal;
+    if (pl.need_gs) { S.x[S.count] = t->grad_student_hidden; S.n[S.count++] = N * H; }
+    if (pl.need_gnw) { S.x[S.count] = t->grad_student_norm_weight; S.n[S.count++] = H; }
+    Timed tm_(ORDA_K_AUX, s, 0.0, 0.0);
+    ORDA_CHECK_LAUNCH(launch_scale<T>(S, s));
+  }
   return ORDA_OK;
 }
 
@@ -1491,7 +1508,7 @@ int orda_gemm(int32_t dtype, int32_t a_mn, int32_t b_mn, int64_t M, int64_t N, i
     if (la != MNMAJ || lb != MNMAJ) return fail(ORDA_EUNSUPPORTED, "split-K is built for MN-major A and B");
     ORDA_TRY(gemm2<T>(la, lb, A, lda, B, ldb, nullptr, 0, K, K, 0, nullptr, part, N, M, N, K, GEMM_SPLIT, sp, kps,
                       s, ORDA_K_AUX, 0.0));
-    ORDA_CHECK_LAUNCH(launch_splitk_reduce<T>(part, sp, M * N, C, ldc, M, N, s));
+    ORDA_CHECK_LAUNCH(launch_splitk_reduce<T>(part, sp, M * N, C, ldc, M, N, nullptr, s));
     return ORDA_OK;
   };
   switch (dtype) {

@@ -1579,6 +1579,14 @@ __device__ __forceinline__ void load4(const T* p, float (&x)[4], bool full, int 
   }
 }
 
+// GemmParams::cscale, for the GEMMs that round to fp16 (1 otherwise: a
+// constant the epilogues' multiplications fold away).
+template <class T>
+__device__ __forceinline__ float gemm_cscale(const GemmParams& P) {
+  if constexpr (std::is_same<T, f16>::value) return P.cscale ? P.cscale[0] : 1.0f;
+  else return 1.0f;
+}
+
 // Epilogue with 4-wide accesses: a lane's 4 consecutive rows of one column
 // are transposed inside the lane quad into 4 consecutive columns of one row
 // (C row-major, ldc a multiple of 4, tile base 8-byte aligned for 16-bit C
@@ -1593,6 +1601,7 @@ __device__ __forceinline__ void gemm_epilogue_q(const f32x16 (&acc)[4][2], const
   float* D = C32 + m0 * P.ldc + n0;
   const int ldc = (int)P.ldc;
   const int mlim = (int)min<int64_t>(P.M - m0, 256), nlim = (int)min<int64_t>(P.N - n0, 256);
+  const float cs = gemm_cscale<T>(P);
   if constexpr (MODE == GEMM_ACC_T && sizeof(T) == 2) {
     if (mlim == 256 && nlim == 256) {
       // interior tile: issue the reads of C for half the tile (two row
@@ -1626,7 +1635,7 @@ __device__ __forceinline__ void gemm_epilogue_q(const f32x16 (&acc)[4][2], const
               union { T e[4]; uint2 u; } v;
               v.u = cv[j][nb][g];
 #pragma unroll
-              for (int e = 0; e < 4; ++e) o[e] += to_f32(v.e[e]);
+              for (int e = 0; e < 4; ++e) o[e] = (o[e] + to_f32(v.e[e])) * cs;
               store4(C + m * ldc + nbase, o, true, 4);
             }
       }
@@ -1651,12 +1660,14 @@ __device__ __forceinline__ void gemm_epilogue_q(const f32x16 (&acc)[4][2], const
           const int off = m * ldc + nbase;
           const bool full = cnt == 4;
           if constexpr (MODE == GEMM_STORE) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] *= cs;
             store4(C + off, o, full, cnt);
           } else if constexpr (MODE == GEMM_ACC_T) {
             float c[4];
             load4(C + off, c, full, cnt);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) c[e] += o[e];
+            for (int e = 0; e < 4; ++e) c[e] = (c[e] + o[e]) * cs;
             store4(C + off, c, full, cnt);
           } else if constexpr (MODE == GEMM_ACC_FIRST || MODE == GEMM_SPLIT) {
             store4(D + off, o, full, cnt);
@@ -1879,6 +1890,7 @@ __global__ __launch_bounds__(kThreads4, 1) void k_gemm4(GemmParams P) {
       return;
     }
     T* C = static_cast<T*>(P.C) + (int64_t)x.m0 * ldc + x.n0;
+    const float cs = gemm_cscale<T>(P);
     const bool wide = sizeof(T) == 2 && ldc % 8 == 0 && reinterpret_cast<uintptr_t>(P.C) % 16 == 0;
     if (mlim == 256 && nlim == 256 && wide) {
       // GEMM_ACC_T: the old values of kRB row blocks (16 kRB rows x 256
@@ -1910,13 +1922,13 @@ __global__ __launch_bounds__(kThreads4, 1) void k_gemm4(GemmParams P) {
             uint4 out;
             if constexpr (MODE == GEMM_ACC_T) {
               const uint4 old = cv[j][pr];
-              out.x = pack2<T>(xv[0] + lo16<T>(old.x), xv[1] + hi16<T>(old.x));
-              out.y = pack2<T>(xv[2] + lo16<T>(old.y), xv[3] + hi16<T>(old.y));
-              out.z = pack2<T>(yv[0] + lo16<T>(old.z), yv[1] + hi16<T>(old.z));
-              out.w = pack2<T>(yv[2] + lo16<T>(old.w), yv[3] + hi16<T>(old.w));
+              out.x = pack2<T>((xv[0] + lo16<T>(old.x)) * cs, (xv[1] + hi16<T>(old.x)) * cs);
+              out.y = pack2<T>((xv[2] + lo16<T>(old.y)) * cs, (xv[3] + hi16<T>(old.y)) * cs);
+              out.z = pack2<T>((yv[0] + lo16<T>(old.z)) * cs, (yv[1] + hi16<T>(old.z)) * cs);
+              out.w = pack2<T>((yv[2] + lo16<T>(old.w)) * cs, (yv[3] + hi16<T>(old.w)) * cs);
             } else {
-              out = make_uint4(pack2<T>(xv[0], xv[1]), pack2<T>(xv[2], xv[3]), pack2<T>(yv[0], yv[1]),
-                               pack2<T>(yv[2], yv[3]));
+              out = make_uint4(pack2<T>(xv[0] * cs, xv[1] * cs), pack2<T>(xv[2] * cs, xv[3] * cs),
+                               pack2<T>(yv[0] * cs, yv[1] * cs), pack2<T>(yv[2] * cs, yv[3] * cs));
             }
             *reinterpret_cast<uint4*>(rp + col16(nb, wn) + cg) = out;
             __builtin_amdgcn_sched_barrier(0);
@@ -1944,6 +1956,8 @@ __global__ __launch_bounds__(kThreads4, 1) void k_gemm4(GemmParams P) {
             for (int e = 0; e < 4; ++e)
               if (e < cnt) o[e] += to_f32(rp[cc + e]);
           }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] *= cs;
           store4(rp + cc, o, cnt == 4 && sizeof(T) == 2 && ldc % 4 == 0, cnt);
         }
       }
@@ -1953,12 +1967,14 @@ __global__ __launch_bounds__(kThreads4, 1) void k_gemm4(GemmParams P) {
                                           tile_info, opnd, epilogue);
 }
 
-// out[m][n] = sum over s of part[s][m][n] (fixed order), converted to T.
+// out[m][n] = sum over s of part[s][m][n] (fixed order), times *scale when
+// given, converted to T.
 // Thread: 4 consecutive columns.  part has leading dimension N (dense),
 // N a multiple of 4.
 template <class T>
 __global__ __launch_bounds__(256) void k_splitk_reduce(const float* __restrict__ part, int splits, int64_t stride,
-                                                       T* __restrict__ out, int64_t ldo, int64_t M, int64_t N) {
+                                                       T* __restrict__ out, int64_t ldo, int64_t M, int64_t N,
+                                                       const float* __restrict__ scale) {
   const int64_t nq = N / 4;
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= M * nq) return;
@@ -1967,6 +1983,11 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(const float* __restrict__
   for (int s = 0; s < splits; ++s) {
     const float4 v = *reinterpret_cast<const float4*>(part + s * stride + m * N + c);
     x[0] += v.x; x[1] += v.y; x[2] += v.z; x[3] += v.w;
+  }
+  if (scale) {
+    const float f = scale[0];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] *= f;
   }
   store4(out + m * ldo + c, x, true, 4);
 }
@@ -3411,10 +3432,10 @@ inline void dlm_go(const DlmParams& P, hipStream_t s) {
   }                                                                                        \
   template <>                                                                              \
   hipError_t launch_splitk_reduce<T>(const float* part, int splits, int64_t stride, void* out, int64_t ldo, \
-                                     int64_t M, int64_t N, hipStream_t s) {                \
+                                     int64_t M, int64_t N, const float* scale, hipStream_t s) { \
     const int64_t n = M * (N / 4);                                                        \
     hipLaunchKernelGGL(k_splitk_reduce<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, part, splits, \
-                       stride, static_cast<T*>(out), ldo, M, N);                           \
+                       stride, static_cast<T*>(out), ldo, M, N, scale);                    \
     return hipGetLastError();                                                              \
   }                                                                                        \
   template <> hipError_t launch_scale<T>(const ScaleParams& P, hipStream_t s) {            \

@@ -91,6 +91,9 @@ struct GemmParams {
   int64_t ldb1, b_kseg, b_kval0, b_kval1;    // valid rows of each segment
   int splits;
   int64_t k_per_split, split_stride;         // split-K (GEMM_SPLIT partials)
+  // fp16 GEMM_STORE / GEMM_ACC_T (k_gemm2, k_gemm4): device scalar that the
+  // fp32 results are multiplied by before they are rounded to C, or null
+  const float* cscale;
 };
 
 // In-place dlogits on materialised logits (k_dlm).
@@ -251,7 +254,7 @@ template <class T> hipError_t launch_rmsnorm_bwd(const NormParams& P, hipStream_
 template <class T> hipError_t launch_two(const TwoParams& P, hipStream_t s);
 template <class T>
 hipError_t launch_splitk_reduce(const float* part, int splits, int64_t stride, void* out, int64_t ldo, int64_t M,
-                                int64_t N, hipStream_t s);
+                                int64_t N, const float* scale, hipStream_t s);
 template <class T> hipError_t launch_scale(const ScaleParams& P, hipStream_t s);
 // out[c * ldo + r] = r < R ? in[r * ldi + c] : 0 for r < Rp, c < C; with in1,
 // the same from in1 to out1 in the same launch

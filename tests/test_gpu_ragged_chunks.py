@@ -7,7 +7,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from tests.test_gpu_parity import _check, _orda, _run
+from tests.test_gpu_parity import _check, _close_grad, _grad_tol, _orda, _run
 
 pytestmark = pytest.mark.gpu
 
@@ -34,8 +34,11 @@ def test_ragged_token_chunks(mode, dtype, V, div, T, N, chunk):
     o = _orda()
     _poison()
     print(f"[ragged] {mode} {dtype} N={N} V={V} chunk={chunk} {div}", flush=True)
-    out, ref, hs, W, _ = _run(
+    out, ref, hs, W, teacher = _run(
         mode, dtype, N=N, H=136, V=V, Ht=None if mode == "tied" else 72, seed=N + V, T=T, div=div,
         w_t=0.5 if mode == "separate" else None, ignore_frac=0.1 if N > 8 else 0.0, w_std=0.1,
         config=o.KernelConfig(chunk_size=chunk) if chunk else None)
     _check(out, ref, hs, W, dtype)
+    if mode == "separate":
+        for got, name in ((teacher.hidden, "grad_teacher_hidden"), (teacher.weight, "grad_teacher_weight")):
+            _close_grad(got.grad, ref[name], name, _grad_tol(dtype))
