@@ -438,6 +438,25 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
         sp = p->grad_hidden_splits;
       } else if (te && cols == pl.H) {
         sp = te->splits_h;
+      } else if (fine && !f32) {
+        // Rule: the least time of rounds of kPersistentGroups 256 x 256 work
+        // items -- 1.4 us per 64-row K step and 10 us of filling the pipeline
+        // and writing out (measured on the ring engine) -- plus the fp32
+        // partials' way out and back at 4 TB/s; at least 512 rows a split.  A
+        // small problem's few tiles spread over more CUs than 16 splits gave
+        // it (256 tokens, hidden 1024, vocabulary 32000, 4 tiles: 54 -> 35 us;
+        // 995 tokens, hidden 384, vocabulary 72448: 219 -> 105).
+        const double tiles = (double)(cdiv(n, 256) * cdiv(cols, 256));
+        double best = 1e30;
+        for (int64_t c = 1; c <= 64 && (c == 1 || pl.V / c >= 512); ++c) {
+          const double rounds = std::ceil(tiles * (double)c / (double)kPersistentGroups);
+          const double cost = rounds * (std::ceil((double)pl.V / (double)c / 64.0) * 1.4 + 10.0) +
+                              (c > 1 ? (double)(c * n * cols) * 8.0 / 4e6 : 0.0);
+          if (cost < best) {
+            best = cost;
+            sp = c;
+          }
+        }
       } else if (f32 && fine) {
         // the least s3_cost over both tile sizes, splits of at least 256 rows
         double best = 1e30;
@@ -539,7 +558,7 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
       pl.fwd_bytes = fo + kAlign;
     };
     layout();
-    if (f32 && pl.fwd_bytes > ORDA_STATIC_SCRATCH_BYTES) {
+    if (pl.fwd_bytes > ORDA_STATIC_SCRATCH_BYTES) {
       // a call that the static entry takes keeps fitting: at most 16 splits
       // (and, in fp32, the vocabulary ranges of 128-token tiles) where more
       // would pass its scratch and those do not
