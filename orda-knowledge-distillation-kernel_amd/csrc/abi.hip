@@ -87,10 +87,12 @@ struct Plan {
   size_t saved_bytes;
   // backward
   bool need_gs, need_gw, need_gt, need_gwt;
-  bool w_dlt_s, w_dlt_t, w_dln_s, w_dln_t, bwd_teacher;
+  bool w_dlt_t, w_dln_t, bwd_student, bwd_teacher;
+  int bwd_splits_s, bwd_splits_t;
+  int64_t bwd_kps_s, bwd_kps_t;
   int bwd_tsrc;
   int64_t NP, ldT, ldh, Vc, nchunks;
-  size_t off_hT, off_htT, off_dLT, off_dLNs, off_dLNt, off_WT, off_WtT, off_g32s, off_g32t, bwd_bytes;
+  size_t off_hT, off_htT, off_dLT, off_bsplit, off_g32s, off_g32t, bwd_bytes;
   // gradients inside forward (materialised token chunks)
   bool fused, store_t, f_tl, f_tmem, f_sring, topk;
   // fp16: dlogits without the mean scale, gradients scaled once at the end
@@ -154,6 +156,45 @@ inline int rule_chunk_scale(const Plan& pl, const orda_problem_t* p, int64_t nco
   if (grads + chunk4 <= kExtraMemoryBudget) return 4;
   const bool out_of_reach = grads + chunk_bytes(n2) > kExtraMemoryBudget;
   return (out_of_reach && chunk4 <= kExtraMemoryBudget) ? 4 : 2;
+}
+
+// Split count of a grad-hidden GEMM (n x cols outputs, K vocabulary rows) by
+// estimated time, up to 64 splits of at least 512 rows (fp32: 256, s3_cost over
+// both tile sizes).  16-bit: rounds of kPersistentGroups 256 x 256 work items,
+// 1.4 us per 64-row K step and 10 us of filling the pipeline and writing out
+// (measured on the ring engine), plus the fp32 partials' way out and back at
+// 4 TB/s.  A small problem's few tiles spread over more CUs than at most 16
+// splits gave it (256 tokens, hidden 1024, vocabulary 32000, 4 tiles: 54 -> 35
+// us; 995 tokens, hidden 384, vocabulary 72448: 219 -> 105).
+inline int64_t splits_by_cost(bool f32, int64_t n, int64_t cols, int64_t K) {
+  int64_t sp = 1;
+  double best = 1e30;
+  const double tiles = (double)(cdiv(n, 256) * cdiv(cols, 256));
+  for (int c = 1; c <= 64 && (c == 1 || K / c >= (f32 ? 256 : 512)); ++c) {
+    double cost;
+    if (f32) {
+      cost = std::min(s3_cost(n, cols, K, c, true), s3_cost(n, cols, K, c, false));
+    } else {
+      const double rounds = std::ceil(tiles * (double)c / (double)kPersistentGroups);
+      cost = rounds * (std::ceil((double)K / (double)c / 64.0) * 1.4 + 10.0) +
+             (c > 1 ? (double)(c * n * cols) * 8.0 / 4e6 : 0.0);
+    }
+    if (cost < best) {
+      best = cost;
+      sp = c;
+    }
+  }
+  return sp;
+}
+
+// Least splits of K rows of `row_bytes` whose K ranges stay inside one 32-bit
+// buffer resource (the ring engine's MN-major operands).
+inline int splits_needed(int64_t row_bytes, int64_t K, int64_t& need) {
+  const int64_t kmax = kRsrcBytes / row_bytes / 64 * 64;
+  if (kmax < 64) return fail(ORDA_EINVAL, "vocab rows of %lld bytes exceed a buffer resource", (long long)row_bytes);
+  need = cdiv(K, kmax);
+  if (need > 64) return fail(ORDA_EINVAL, "grad hidden needs %lld splits of the vocabulary (at most 64)", (long long)need);
+  return ORDA_OK;
 }
 
 int make_plan(const orda_problem_t* p, Plan& pl) {
@@ -302,40 +343,44 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
   pl.need_gt = (f & ORDA_NEED_GRAD_TEACHER_HIDDEN) != 0 && (tied || sep);
   pl.need_gwt = (f & ORDA_NEED_GRAD_TEACHER_WEIGHT) != 0 && sep;
   const bool tgrad = pl.teacher_ce && (tied || sep);
-  pl.w_dlt_s = pl.need_gw;
-  pl.w_dln_s = pl.need_gs;
   pl.w_dlt_t = tgrad && ((tied && pl.need_gw) || (sep && pl.need_gwt));
   pl.w_dln_t = tgrad && pl.need_gt;
+  pl.bwd_student = pl.need_gs || pl.need_gw;
   pl.bwd_teacher = pl.w_dlt_t || pl.w_dln_t;
   pl.bwd_tsrc = (pl.div_on || pl.bwd_teacher) ? pl.tsrc : TSRC_NONE;
   if (pl.bwd_teacher && pl.tsrc == TSRC_NONE) pl.bwd_tsrc = tied ? TSRC_SHARED : TSRC_SEP;
   pl.NP = round_up(pl.N, 8);
-  pl.ldT = pl.w_dlt_t ? 2 * pl.NP : pl.NP;
+  pl.ldT = pl.bwd_teacher ? 2 * pl.NP : pl.NP;
   pl.ldh = (tied && pl.w_dlt_t) ? 2 * pl.NP : pl.NP;
+  // one vocabulary chunk's dlogits are staged vocabulary-major ([Vc][ldT],
+  // read by grad W as its K-major and by grad hidden as its MN-major operand)
   const int64_t Vmax = round_up(pl.V, 256);
-  int64_t per_col = 0;
-  if (pl.w_dlt_s || pl.w_dlt_t) per_col += pl.ldT;
-  if (pl.w_dln_s) per_col += pl.N;
-  if (pl.w_dln_t) per_col += pl.N;
-  if (pl.need_gs || (tied && pl.w_dln_t)) per_col += pl.H;
-  if (sep && pl.w_dln_t) per_col += pl.Ht;
-  per_col *= pl.eb;
+  const int64_t per_col = pl.ldT * pl.eb;
   if (p->vocab_chunk > 0) {
     pl.Vc = round_up(p->vocab_chunk, 256);
   } else {
-    pl.Vc = per_col > 0 ? (kDefaultStagingBytes / per_col) / 256 * 256 : Vmax;
+    pl.Vc = (kDefaultStagingBytes / per_col) / 256 * 256;
   }
   if (pl.Vc < 256) pl.Vc = 256;
   if (pl.Vc > Vmax) pl.Vc = Vmax;
   pl.nchunks = cdiv(pl.V, pl.Vc);
+  auto bwd_split = [&](int64_t cols, int& splits, int64_t& kps) -> int {
+    int64_t sp = splits_by_cost(f32, pl.N, cols, std::min(pl.Vc, pl.V));
+    int64_t need = 1;
+    ORDA_TRY_PLAN(splits_needed(std::max(pl.ldT, cols) * pl.eb, pl.Vc, need));
+    if (sp < need) sp = need;
+    kps = round_up(cdiv(pl.Vc, sp), 64);
+    splits = (int)cdiv(pl.Vc, kps);
+    return ORDA_OK;
+  };
+  ORDA_TRY_PLAN(bwd_split(pl.H, pl.bwd_splits_s, pl.bwd_kps_s));
+  ORDA_TRY_PLAN(bwd_split(pl.Ht > 0 ? pl.Ht : pl.H, pl.bwd_splits_t, pl.bwd_kps_t));
   off = 0;
-  pl.off_hT = pl.need_gw ? carve(off, (size_t)pl.H * pl.ldh * pl.eb) : 0;
-  pl.off_htT = (sep && pl.w_dlt_t) ? carve(off, (size_t)pl.Ht * pl.NP * pl.eb) : 0;
-  pl.off_dLT = (pl.w_dlt_s || pl.w_dlt_t) ? carve(off, (size_t)pl.Vc * pl.ldT * pl.eb) : 0;
-  pl.off_dLNs = pl.w_dln_s ? carve(off, (size_t)pl.N * pl.Vc * pl.eb) : 0;
-  pl.off_dLNt = pl.w_dln_t ? carve(off, (size_t)pl.N * pl.Vc * pl.eb) : 0;
-  pl.off_WT = (pl.need_gs || (tied && pl.w_dln_t)) ? carve(off, (size_t)pl.H * pl.Vc * pl.eb) : 0;
-  pl.off_WtT = (sep && pl.w_dln_t) ? carve(off, (size_t)pl.Ht * pl.Vc * pl.eb) : 0;
+  pl.off_hT = (pl.need_gw && !f32) ? carve(off, (size_t)pl.H * pl.ldh * pl.eb) : 0;
+  pl.off_htT = (sep && pl.w_dlt_t && !f32) ? carve(off, (size_t)pl.Ht * pl.NP * pl.eb) : 0;
+  pl.off_dLT = (pl.bwd_student || pl.bwd_teacher) ? carve(off, (size_t)pl.Vc * pl.ldT * pl.eb) : 0;
+  const int64_t part_s = pl.need_gs ? pl.bwd_splits_s * pl.H : 0, part_t = pl.w_dln_t ? pl.bwd_splits_t * pl.Ht : 0;
+  pl.off_bsplit = carve(off, (size_t)std::max(part_s, part_t) * pl.N * 4);
   pl.off_g32s = (pl.need_gs && pl.nchunks > 1) ? carve(off, (size_t)pl.N * pl.H * 4) : 0;
   pl.off_g32t = (pl.w_dln_t && pl.nchunks > 1) ? carve(off, (size_t)pl.N * pl.Ht * 4) : 0;
   pl.bwd_bytes = off + kAlign;
@@ -438,35 +483,8 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
         sp = p->grad_hidden_splits;
       } else if (te && cols == pl.H) {
         sp = te->splits_h;
-      } else if (fine && !f32) {
-        // Rule: the least time of rounds of kPersistentGroups 256 x 256 work
-        // items -- 1.4 us per 64-row K step and 10 us of filling the pipeline
-        // and writing out (measured on the ring engine) -- plus the fp32
-        // partials' way out and back at 4 TB/s; at least 512 rows a split.  A
-        // small problem's few tiles spread over more CUs than 16 splits gave
-        // it (256 tokens, hidden 1024, vocabulary 32000, 4 tiles: 54 -> 35 us;
-        // 995 tokens, hidden 384, vocabulary 72448: 219 -> 105).
-        const double tiles = (double)(cdiv(n, 256) * cdiv(cols, 256));
-        double best = 1e30;
-        for (int64_t c = 1; c <= 64 && (c == 1 || pl.V / c >= 512); ++c) {
-          const double rounds = std::ceil(tiles * (double)c / (double)kPersistentGroups);
-          const double cost = rounds * (std::ceil((double)pl.V / (double)c / 64.0) * 1.4 + 10.0) +
-                              (c > 1 ? (double)(c * n * cols) * 8.0 / 4e6 : 0.0);
-          if (cost < best) {
-            best = cost;
-            sp = c;
-          }
-        }
-      } else if (f32 && fine) {
-        // the least s3_cost over both tile sizes, splits of at least 256 rows
-        double best = 1e30;
-        for (int c = 1; c <= 64 && (c == 1 || pl.V / c >= 256); ++c) {
-          const double cost = std::min(s3_cost(n, cols, pl.V, c, true), s3_cost(n, cols, pl.V, c, false));
-          if (cost < best) {
-            best = cost;
-            sp = c;
-          }
-        }
+      } else if (fine) {
+        sp = splits_by_cost(f32, n, cols, pl.V);
       } else {
         // Rule: the persistent GEMM runs its tiles x splits equal work items
         // in rounds of kPersistentGroups workgroups, so its time goes as
@@ -487,14 +505,9 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
           }
         }
       }
-      // each split's K range of both MN-major operands (the chunk's dlogits,
-      // ld = fldL, and the weight, ld = cols) must stay inside one 32-bit
-      // buffer resource
-      const int64_t ldmax = std::max<int64_t>(pl.fldL, cols) * pl.eb;
-      const int64_t kmax = kRsrcBytes / ldmax / 64 * 64;
-      if (kmax < 64) return fail(ORDA_EINVAL, "vocab rows of %lld bytes exceed a buffer resource", (long long)ldmax);
-      const int64_t need = cdiv(pl.V, kmax);
-      if (need > 64) return fail(ORDA_EINVAL, "grad hidden needs %lld splits of the vocabulary (at most 64)", (long long)need);
+      // (the chunk's dlogits, ld = fldL, and the weight, ld = cols)
+      int64_t need = 1;
+      ORDA_TRY_PLAN(splits_needed(std::max<int64_t>(pl.fldL, cols) * pl.eb, pl.V, need));
       if (sp < need) sp = need;
       kps = round_up(cdiv(pl.V, sp), 64);
       splits = (int)cdiv(pl.V, kps);
@@ -744,122 +757,6 @@ int scale_grads(const Plan& pl, const orda_tensors_t* t, const float* factor, hi
   return ORDA_OK;
 }
 
-template <class T>
-int run_backward(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, char* ws, hipStream_t s) {
-  const bool tied = pl.mode == ORDA_MODE_TIED, sep = pl.mode == ORDA_MODE_SEPARATE;
-  const int eb = pl.eb;
-  const int64_t N = pl.N, H = pl.H, Ht = pl.Ht, NP = pl.NP;
-  char* hT = ws + pl.off_hT;
-  char* htT = ws + pl.off_htT;
-  char* dLT = ws + pl.off_dLT;
-  char* dLNs = ws + pl.off_dLNs;
-  char* dLNt = ws + pl.off_dLNt;
-  char* WT = ws + pl.off_WT;
-  char* WtT = ws + pl.off_WtT;
-  float* g32s = reinterpret_cast<float*>(ws + pl.off_g32s);
-  float* g32t = reinterpret_cast<float*>(ws + pl.off_g32t);
-  float* scal = static_cast<float*>(t->saved);
-  float* rowp = scal + kScalFloats;
-
-  // Tied mode with teacher CE off: the teacher hidden gradient is zero
-  // (reference ops/tied_teacher.py:478-479).
-  if (tied && pl.need_gt && !pl.w_dln_t)
-    { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(t->grad_teacher_hidden, H, N, 0, H, eb, s)); }
-
-  const bool any = pl.w_dlt_s || pl.w_dlt_t || pl.w_dln_s || pl.w_dln_t;
-  if (!any) return ORDA_OK;
-
-  // Transposed hidden states for the grad_W GEMMs (K = tokens), with zeroed
-  // padding columns so K can be rounded up to a multiple of 8.
-  if (pl.need_gw) {
-    const bool both = tied && pl.w_dlt_t;
-    Timed tm_(ORDA_K_AUX, s, 0.0, 0.0);
-    ORDA_CHECK_LAUNCH(launch_transpose<T>(t->student_hidden, H, hT, pl.ldh, N, NP, H, s,
-                                          both ? t->teacher_hidden : nullptr, both ? hT + NP * eb : nullptr));
-  }
-  if (sep && pl.w_dlt_t)
-    { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(t->teacher_hidden, Ht, htT, NP, N, NP, Ht, s)); }
-  // padding columns of the staged dlogits (never written by the dL kernel)
-  if (pl.w_dlt_s || pl.w_dlt_t) { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(dLT, pl.ldT, pl.Vc, N, NP, eb, s)); }
-  if (pl.w_dlt_t) { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(dLT, pl.ldT, pl.Vc, NP + N, 2 * NP, eb, s)); }
-
-  FusedParams F{};
-  F.W = t->weight; F.hs = t->student_hidden; F.ht = t->teacher_hidden; F.Wt = t->teacher_weight;
-  F.Lt = t->teacher_logits; F.labels = t->labels;
-  F.N = N; F.V = pl.V; F.H = H; F.Ht = Ht; F.ignore_index = p->ignore_index;
-  F.tsrc = pl.bwd_tsrc; F.lt_dtype = p->logits_dtype;
-  F.div = pl.div; F.fam = pl.fam; F.t_is_one = pl.t1; F.tgrad = pl.bwd_teacher;
-  F.temperature = p->temperature; F.invT = 1.0f / p->temperature;
-  F.alpha = p->div_alpha; F.beta = p->div_beta;
-  set_mix(F.mix_w, F.mix_w1, p);
-  const int n_ttiles = (int)cdiv(N, 128);  // k_dl's
-  F.n_ttiles = n_ttiles; F.rowp = rowp;
-  F.w_s = p->student_ce_weight; F.w_t = p->teacher_ce_weight; F.w_kl = pl.div_on ? p->kl_weight : 0.f;
-  // fp16: unscaled dlogits (scal[2] = 1); the gradients get grad_output x
-  // mean_scale at the end
-  F.grad_output = pl.late_scale ? scal + 2 : t->grad_output;
-  F.mean_scale = pl.late_scale ? scal + 2 : scal;
-  F.dLT = dLT; F.ldT = pl.ldT; F.tcol = NP; F.dLNs = dLNs; F.dLNt = dLNt; F.ldN = pl.Vc;
-  F.w_dlt_s = pl.w_dlt_s; F.w_dlt_t = pl.w_dlt_t; F.w_dln_s = pl.w_dln_s; F.w_dln_t = pl.w_dln_t;
-
-  const int64_t Kw = (tied && pl.w_dlt_t) ? 2 * NP : NP;
-  for (int64_t c = 0; c < pl.nchunks; ++c) {
-    const int64_t vc0 = c * pl.Vc;
-    const int64_t vcc = (pl.V - vc0 < pl.Vc) ? pl.V - vc0 : pl.Vc;
-    const int64_t vck = round_up(vcc, pl.kelems);  // K of the grad_hidden GEMMs
-    const int gmode = pl.nchunks == 1 ? GEMM_STORE
-                      : c == 0 ? GEMM_ACC_FIRST
-                      : c == pl.nchunks - 1 ? GEMM_ACC_LAST : GEMM_ACC;
-    const bool needWT = pl.need_gs || (tied && pl.w_dln_t);
-    if (needWT) {
-      { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(static_cast<const char*>(t->weight) + vc0 * H * eb, H, WT, pl.Vc, vcc, vck, H, s)); }
-    }
-    if (sep && pl.w_dln_t) {
-      { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(static_cast<const char*>(t->teacher_weight) + vc0 * Ht * eb, Ht, WtT, pl.Vc, vcc, vck, Ht, s)); }
-    }
-    if (vck > vcc) {
-      if (pl.w_dln_s) { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(dLNs, pl.Vc, N, vcc, vck, eb, s)); }
-      if (pl.w_dln_t) { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(dLNt, pl.Vc, N, vcc, vck, eb, s)); }
-    }
-    F.vc0 = vc0; F.vcc = vcc;
-    const int grid = (int)(cdiv(vcc, 256) * n_ttiles);
-    {
-      const double kt = (pl.bwd_tsrc == TSRC_SHARED || pl.bwd_tsrc == TSRC_SEP) ? (double)Ht : 0.0;
-      Timed tm_(ORDA_K_DLOGITS, s, 0.0, 2.0 * (double)N * (double)vcc * ((double)H + kt));
-      ORDA_CHECK_LAUNCH(launch_dl<T>(F, grid, s));
-    }
-
-    if (pl.need_gw) {
-      const double kv = (tied && pl.w_dlt_t) ? 2.0 * (double)N : (double)N;
-      ORDA_TRY(gemm<T>(dLT, pl.ldT, hT, pl.ldh, static_cast<char*>(t->grad_weight) + vc0 * H * eb, nullptr, H, vcc,
-                       H, Kw, GEMM_STORE, s, ORDA_K_GEMM_W, 2.0 * (double)vcc * (double)H * kv));
-    }
-    if (sep && pl.need_gwt && pl.w_dlt_t) {
-      ORDA_TRY(gemm<T>(dLT + NP * eb, pl.ldT, htT, NP, static_cast<char*>(t->grad_teacher_weight) + vc0 * Ht * eb,
-                       nullptr, Ht, vcc, Ht, NP, GEMM_STORE, s, ORDA_K_GEMM_W,
-                       2.0 * (double)vcc * (double)Ht * (double)N));
-    }
-    if (pl.need_gs) {
-      ORDA_TRY(gemm<T>(dLNs, pl.Vc, WT, pl.Vc, t->grad_student_hidden, g32s, H, N, H, vck, gmode, s, ORDA_K_GEMM_H,
-                       2.0 * (double)N * (double)H * (double)vcc));
-    }
-    if (pl.w_dln_t) {
-      ORDA_TRY(gemm<T>(dLNt, pl.Vc, tied ? WT : WtT, pl.Vc, t->grad_teacher_hidden, g32t, Ht, N, Ht, vck, gmode, s,
-                       ORDA_K_GEMM_H, 2.0 * (double)N * (double)Ht * (double)vcc));
-    }
-  }
-  // separate mode, teacher weight grad requested but teacher CE off: zero
-  if (sep && pl.need_gwt && !pl.w_dlt_t)
-    { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(t->grad_teacher_weight, Ht, pl.V, 0, Ht, eb, s)); }
-  if (sep && pl.need_gt && !pl.w_dln_t)
-    { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(t->grad_teacher_hidden, Ht, N, 0, Ht, eb, s)); }
-  if (pl.late_scale) {
-    { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_mul_scalars(t->grad_output, scal, scal + 3, s)); }
-    ORDA_TRY(scale_grads<T>(pl, t, scal + 3, s));
-  }
-  return ORDA_OK;
-}
-
 // One launch of the general GEMM (k_gemm2); B1/b_kseg/b_kval* describe an
 // MN-major B in two row segments (b_kseg = K, b_kval0 = K, B1 = NULL for
 // one).  splits > 1 writes fp32 partials [splits][M][N] to C32 (mode SPLIT).
@@ -894,6 +791,132 @@ inline int gemm_s3(int la, int lb, const void* A, int64_t lda, const void* B, co
   G.splits = splits; G.k_per_split = splits > 1 ? kps : K; G.split_stride = M * ldc;
   Timed tm_(kind, s, alg, 2.0 * (double)M * (double)N * (double)K);
   ORDA_CHECK_LAUNCH(launch_gemm_s3(G, s));
+  return ORDA_OK;
+}
+
+// Two-phase backward: per vocabulary chunk the dlogits (k_dl recomputes the
+// logits), grad W's rows (one fp32-accumulated GEMM over all tokens, rounded
+// once) and grad hidden's share (both operands MN-major, split over the
+// chunk's rows; the partials are added up in fp32, over the chunks too).  The
+// GEMMs are the ring engine's (fp32: the split-operand engine's): at 4096
+// tokens, hidden 2048, vocabulary 100277 they took 5.1 ms a step on the
+// two-stage engine with a token-major copy of the dlogits and a transposed
+// copy of W.
+template <class T>
+int run_backward(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t, char* ws, hipStream_t s) {
+  const bool tied = pl.mode == ORDA_MODE_TIED, sep = pl.mode == ORDA_MODE_SEPARATE;
+  const int eb = pl.eb;
+  const int64_t N = pl.N, H = pl.H, Ht = pl.Ht, NP = pl.NP;
+  char* hT = ws + pl.off_hT;
+  char* htT = ws + pl.off_htT;
+  char* dLT = ws + pl.off_dLT;
+  float* bsplit = reinterpret_cast<float*>(ws + pl.off_bsplit);
+  float* g32s = reinterpret_cast<float*>(ws + pl.off_g32s);
+  float* g32t = reinterpret_cast<float*>(ws + pl.off_g32t);
+  float* scal = static_cast<float*>(t->saved);
+  float* rowp = scal + kScalFloats;
+
+  // Tied mode with teacher CE off: the teacher hidden gradient is zero
+  // (reference ops/tied_teacher.py:478-479).
+  if (tied && pl.need_gt && !pl.w_dln_t)
+    { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(t->grad_teacher_hidden, H, N, 0, H, eb, s)); }
+  // separate mode, teacher gradients requested but teacher CE off: zero
+  if (sep && pl.need_gwt && !pl.w_dlt_t)
+    { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(t->grad_teacher_weight, Ht, pl.V, 0, Ht, eb, s)); }
+  if (sep && pl.need_gt && !pl.w_dln_t)
+    { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(t->grad_teacher_hidden, Ht, N, 0, Ht, eb, s)); }
+  if (!pl.bwd_student && !pl.bwd_teacher) return ORDA_OK;
+
+  // 16-bit: transposed hidden states for the grad_W GEMMs (K = tokens), with
+  // zeroed padding columns so K can be rounded up to a multiple of 8
+  const bool both = tied && pl.w_dlt_t;
+  if (pl.need_gw && eb == 2) {
+    Timed tm_(ORDA_K_AUX, s, 0.0, 0.0);
+    ORDA_CHECK_LAUNCH(launch_transpose<T>(t->student_hidden, H, hT, pl.ldh, N, NP, H, s,
+                                          both ? t->teacher_hidden : nullptr, both ? hT + NP * eb : nullptr));
+  }
+  if (sep && pl.w_dlt_t && eb == 2)
+    { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_transpose<T>(t->teacher_hidden, Ht, htT, NP, N, NP, Ht, s)); }
+  // padding columns of the staged dlogits (never written by the dL kernel)
+  { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(dLT, pl.ldT, pl.Vc, N, NP, eb, s)); }
+  if (pl.bwd_teacher) { Timed tm_(ORDA_K_AUX, s, 0.0, 0.0); ORDA_CHECK_LAUNCH(launch_zero2d(dLT, pl.ldT, pl.Vc, NP + N, 2 * NP, eb, s)); }
+  // fp16: unscaled dlogits (scal[2] = 1); grad_output x mean_scale goes into
+  // the gradient GEMMs' last rounding
+  const float* late = nullptr;
+  if (pl.late_scale) {
+    Timed tm_(ORDA_K_AUX, s, 0.0, 0.0);
+    ORDA_CHECK_LAUNCH(launch_mul_scalars(t->grad_output, scal, scal + 3, s));
+    late = scal + 3;
+  }
+
+  FusedParams F{};
+  F.W = t->weight; F.hs = t->student_hidden; F.ht = t->teacher_hidden; F.Wt = t->teacher_weight;
+  F.Lt = t->teacher_logits; F.labels = t->labels;
+  F.N = N; F.V = pl.V; F.H = H; F.Ht = Ht; F.ignore_index = p->ignore_index;
+  F.tsrc = pl.bwd_tsrc; F.lt_dtype = p->logits_dtype;
+  F.div = pl.div; F.fam = pl.fam; F.t_is_one = pl.t1; F.tgrad = pl.bwd_teacher;
+  F.temperature = p->temperature; F.invT = 1.0f / p->temperature;
+  F.alpha = p->div_alpha; F.beta = p->div_beta;
+  set_mix(F.mix_w, F.mix_w1, p);
+  F.n_ttiles = (int)cdiv(N, 128); F.rowp = rowp;
+  F.w_s = p->student_ce_weight; F.w_t = p->teacher_ce_weight; F.w_kl = pl.div_on ? p->kl_weight : 0.f;
+  F.grad_output = pl.late_scale ? scal + 2 : t->grad_output;
+  F.mean_scale = pl.late_scale ? scal + 2 : scal;
+  F.dLT = dLT; F.ldT = pl.ldT; F.tcol = NP;
+  F.w_dlt_s = pl.bwd_student; F.w_dlt_t = pl.bwd_teacher;
+
+  for (int64_t c = 0; c < pl.nchunks; ++c) {
+    const int64_t vc0 = c * pl.Vc;
+    const int64_t vcc = (pl.V - vc0 < pl.Vc) ? pl.V - vc0 : pl.Vc;
+    const T* W = static_cast<const T*>(t->weight) + vc0 * H;
+    const T* Wt = t->teacher_weight ? static_cast<const T*>(t->teacher_weight) + vc0 * Ht : nullptr;
+    F.vc0 = vc0; F.vcc = vcc;
+    {
+      const double kt = (pl.bwd_tsrc == TSRC_SHARED || pl.bwd_tsrc == TSRC_SEP) ? (double)Ht : 0.0;
+      Timed tm_(ORDA_K_DLOGITS, s, 0.0, 2.0 * (double)N * (double)vcc * ((double)H + kt));
+      ORDA_CHECK_LAUNCH(launch_dl<T>(F, (int)(cdiv(vcc, 256) * F.n_ttiles), s));
+    }
+    // grad W rows [vc0, vc0 + vcc) = dL^T [hs; ht]
+    auto grad_w = [&](const char* A, const void* h, const void* h1, const char* hTx, int64_t ldh, int64_t cols,
+                      void* dst, int64_t K) -> int {
+      void* out = static_cast<T*>(dst) + vc0 * cols;
+      const double fl = 2.0 * (double)vcc * (double)cols * (double)N * (h1 ? 2.0 : 1.0);
+      if constexpr (sizeof(T) == 4)
+        return gemm_s3(KMAJ, MNMAJ, A, pl.ldT, h, h1, cols, NP, N, N, out, nullptr, cols, vcc, cols, K, GEMM_STORE, 1, 0,
+                       s, ORDA_K_GEMM_W, fl);
+      else
+        return gemm2<T>(KMAJ, KMAJ, A, pl.ldT, hTx, ldh, nullptr, 0, K, K, 0, out, nullptr, cols, vcc, cols, K,
+                        GEMM_STORE, 1, 0, s, ORDA_K_GEMM_W, fl, late);
+    };
+    if (pl.need_gw)
+      ORDA_TRY(grad_w(dLT, t->student_hidden, both ? t->teacher_hidden : nullptr, hT, pl.ldh, H, t->grad_weight,
+                      both ? 2 * NP : NP));
+    if (sep && pl.need_gwt && pl.w_dlt_t)
+      ORDA_TRY(grad_w(dLT + NP * eb, t->teacher_hidden, nullptr, htT, NP, Ht, t->grad_teacher_weight, NP));
+    // grad hidden (+)= dL W
+    const int gmode = pl.nchunks == 1 ? GEMM_STORE
+                      : c == 0 ? GEMM_ACC_FIRST
+                      : c == pl.nchunks - 1 ? GEMM_ACC_LAST : GEMM_ACC;
+    auto grad_hidden = [&](const char* A, const T* Wx, int64_t cols, void* dst, float* g32, int splits,
+                           int64_t kps) -> int {
+      const double fl = 2.0 * (double)N * (double)cols * (double)vcc;
+      const int sp = (int)std::min<int64_t>(splits, cdiv(vcc, kps));  // (a short last chunk has fewer)
+      if constexpr (sizeof(T) == 4)
+        ORDA_TRY(gemm_s3(MNMAJ, MNMAJ, A, pl.ldT, Wx, nullptr, cols, 0, vcc, 0, nullptr, bsplit, cols, N, cols, vcc,
+                         GEMM_SPLIT, sp, kps, s, ORDA_K_GEMM_H, fl));
+      else
+        ORDA_TRY(gemm2<T>(MNMAJ, MNMAJ, A, pl.ldT, Wx, cols, nullptr, 0, vcc, vcc, 0, nullptr, bsplit, cols, N, cols,
+                          vcc, GEMM_SPLIT, sp, kps, s, ORDA_K_GEMM_H, fl));
+      Timed tm_(ORDA_K_AUX, s, 0.0, 0.0);
+      ORDA_CHECK_LAUNCH(launch_splitk_reduce<T>(bsplit, sp, N * cols, dst, cols, N, cols, late, s, g32, gmode));
+      return ORDA_OK;
+    };
+    if (pl.need_gs)
+      ORDA_TRY(grad_hidden(dLT, W, H, t->grad_student_hidden, g32s, pl.bwd_splits_s, pl.bwd_kps_s));
+    if (pl.w_dln_t)
+      ORDA_TRY(grad_hidden(dLT + NP * eb, tied ? W : Wt, Ht, t->grad_teacher_hidden, g32t, pl.bwd_splits_t,
+                           pl.bwd_kps_t));
+  }
   return ORDA_OK;
 }
 

@@ -1415,8 +1415,6 @@ __device__ __forceinline__ void dl_tile(const f32x16 (&acc)[4][2], const FusedPa
   const float invT = P.invT;
   const int64_t vend = min(P.V, P.vc0 + P.vcc);
   T* dLT = static_cast<T*>(P.dLT);
-  T* dLNs = static_cast<T*>(P.dLNs);
-  T* dLNt = static_cast<T*>(P.dLNt);
   const int64_t y = P.labels[tr];
   const bool ignored = !tok_ok || (y == P.ignore_index);
   const int64_t yeff = (y >= 0 && y < P.V) ? y : 0;
@@ -1461,13 +1459,9 @@ __device__ __forceinline__ void dl_tile(const f32x16 (&acc)[4][2], const FusedPa
         }
       }
       const int64_t vl = vg - P.vc0;  // row inside the chunk
-      const bool rows_full = vg + 3 < vend;
-      // token-major staging: this lane's 4 consecutive rows are contiguous
-      if (P.w_dln_s && tok_ok) store4(dLNs + t * P.ldN + vl, gs, rows_full, (int)(vend - vg));
-      if (P.w_dln_t && tok_ok) store4(dLNt + t * P.ldN + vl, gt, rows_full, (int)(vend - vg));
-      // row-major staging: transpose inside the lane quad so each lane
+      // vocabulary-major staging: transpose inside the lane quad so each lane
       // holds 4 consecutive tokens of one row
-      if (P.w_dlt_s || P.w_dlt_t) {
+      {
         const int q = lane & 3;
         const int64_t tb = t - q;  // first token of the quad
         const int ntok = (int)min<int64_t>(P.N - tb, 4);
@@ -1968,13 +1962,15 @@ __global__ __launch_bounds__(kThreads4, 1) void k_gemm4(GemmParams P) {
 }
 
 // out[m][n] = sum over s of part[s][m][n] (fixed order), times *scale when
-// given, converted to T.
-// Thread: 4 consecutive columns.  part has leading dimension N (dense),
-// N a multiple of 4.
+// given, converted to T.  Thread: 4 consecutive columns.  part has leading
+// dimension N (dense), N a multiple of 4.  With acc (dense [M x N] fp32) the
+// sum goes on over calls: `mode` GEMM_ACC_FIRST writes it to acc, GEMM_ACC
+// adds to acc, GEMM_ACC_LAST adds acc and writes out; GEMM_STORE has no acc.
 template <class T>
 __global__ __launch_bounds__(256) void k_splitk_reduce(const float* __restrict__ part, int splits, int64_t stride,
                                                        T* __restrict__ out, int64_t ldo, int64_t M, int64_t N,
-                                                       const float* __restrict__ scale) {
+                                                       const float* __restrict__ scale, float* __restrict__ acc,
+                                                       int mode) {
   const int64_t nq = N / 4;
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= M * nq) return;
@@ -1983,6 +1979,14 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(const float* __restrict__
   for (int s = 0; s < splits; ++s) {
     const float4 v = *reinterpret_cast<const float4*>(part + s * stride + m * N + c);
     x[0] += v.x; x[1] += v.y; x[2] += v.z; x[3] += v.w;
+  }
+  if (mode == GEMM_ACC || mode == GEMM_ACC_LAST) {
+    const float4 v = *reinterpret_cast<const float4*>(acc + m * N + c);
+    x[0] += v.x; x[1] += v.y; x[2] += v.z; x[3] += v.w;
+  }
+  if (mode == GEMM_ACC_FIRST || mode == GEMM_ACC) {
+    *reinterpret_cast<float4*>(acc + m * N + c) = make_float4(x[0], x[1], x[2], x[3]);
+    return;
   }
   if (scale) {
     const float f = scale[0];
@@ -3432,10 +3436,10 @@ inline void dlm_go(const DlmParams& P, hipStream_t s) {
   }                                                                                        \
   template <>                                                                              \
   hipError_t launch_splitk_reduce<T>(const float* part, int splits, int64_t stride, void* out, int64_t ldo, \
-                                     int64_t M, int64_t N, const float* scale, hipStream_t s) { \
+                                     int64_t M, int64_t N, const float* scale, hipStream_t s, float* acc, int mode) { \
     const int64_t n = M * (N / 4);                                                        \
     hipLaunchKernelGGL(k_splitk_reduce<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, part, splits, \
-                       stride, static_cast<T*>(out), ldo, M, N, scale);                    \
+                       stride, static_cast<T*>(out), ldo, M, N, scale, acc, mode);         \
     return hipGetLastError();                                                              \
   }                                                                                        \
   template <> hipError_t launch_scale<T>(const ScaleParams& P, hipStream_t s) {            \

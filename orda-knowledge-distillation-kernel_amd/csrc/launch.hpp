@@ -56,10 +56,7 @@ struct FusedParams {
   const float* mean_scale;
   void* dLT;
   int64_t ldT, tcol;
-  void* dLNs;
-  void* dLNt;
-  int64_t ldN;
-  int w_dlt_s, w_dlt_t, w_dln_s, w_dln_t;
+  int w_dlt_s, w_dlt_t;
   // logits written by the scan of the materialised path: Lout[v][t],
   // teacher columns from tcolL (stored when store_t)
   void* Lout;
@@ -254,7 +251,8 @@ template <class T> hipError_t launch_rmsnorm_bwd(const NormParams& P, hipStream_
 template <class T> hipError_t launch_two(const TwoParams& P, hipStream_t s);
 template <class T>
 hipError_t launch_splitk_reduce(const float* part, int splits, int64_t stride, void* out, int64_t ldo, int64_t M,
-                                int64_t N, const float* scale, hipStream_t s);
+                                int64_t N, const float* scale, hipStream_t s, float* acc = nullptr,
+                                int mode = GEMM_STORE);
 template <class T> hipError_t launch_scale(const ScaleParams& P, hipStream_t s);
 // out[c * ldo + r] = r < R ? in[r * ldi + c] : 0 for r < Rp, c < C; with in1,
 // the same from in1 to out1 in the same launch
