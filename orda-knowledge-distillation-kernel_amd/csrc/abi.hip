@@ -82,6 +82,7 @@ struct Plan {
   int tsrc, div, fam, npow;
   float pa[3], pb[3];
   // forward
+  bool fwd_ring;
   int f_tok, n_ttiles, n_vtiles, n_vranges, tiles_per_range;
   size_t off_partial, off_labelx, off_rowv, fwd_bytes;
   size_t saved_bytes;
@@ -322,7 +323,17 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
   const bool f32 = p->dtype == ORDA_F32;
   pl.n_ttiles = (int)cdiv(pl.N, f32 && (pl.tsrc == TSRC_SHARED || pl.tsrc == TSRC_SEP) ? 64 : 128);
   pl.n_vtiles = (int)cdiv(pl.V, 256);
-  int64_t nvr = f32 ? kPersistentGroups / pl.n_ttiles : cdiv(kScanTargetGroups, pl.n_ttiles);  // two-phase scan
+  // 16-bit without a teacher's GEMM beside the student's: the ring engine's
+  // student-only tiles of 256 tokens, teacher logits of the compute dtype read
+  // in place (three power terms per token would spill there).  The two-stage
+  // engine's lanes read single teacher logits: 4096 tokens, hidden 4096,
+  // vocabulary 128256 with cached logits, losses only, 3.3 ms on the ring
+  // (7.5 with the gradients that a no_grad call used to compute).
+  const bool ring_mem = pl.tsrc == TSRC_MEM && p->logits_dtype == p->dtype && pl.V % 4 == 0 &&
+                        pl.V <= 65535 * 64 && !(pl.fam == FAM_POW && pl.npow != 1);
+  pl.fwd_ring = !f32 && pl.H > 64 && (pl.tsrc == TSRC_NONE || ring_mem);
+  if (pl.fwd_ring) pl.n_ttiles = (int)cdiv(pl.N, 256);
+  int64_t nvr = (f32 || pl.fwd_ring) ? kPersistentGroups / pl.n_ttiles : cdiv(kScanTargetGroups, pl.n_ttiles);  // two-phase scan
   if (nvr < 1) nvr = 1;
   if (nvr > pl.n_vtiles) nvr = pl.n_vtiles;
   pl.tiles_per_range = (int)cdiv(pl.n_vtiles, nvr);
@@ -685,7 +696,16 @@ int run_forward(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t
   F.phase = 0; F.n_ttiles = pl.n_ttiles; F.n_vranges = pl.n_vranges;
   F.tiles_per_range = pl.tiles_per_range; F.n_vtiles = pl.n_vtiles;
   F.partial = partial; F.rowp = rowp;
-  const int grid = pl.n_ttiles * pl.n_vranges;
+  int grid = pl.n_ttiles * pl.n_vranges;
+  if (pl.fwd_ring) {
+    F.student_ring = pl.tsrc == TSRC_NONE;
+    if (pl.tsrc == TSRC_MEM && reinterpret_cast<uintptr_t>(t->teacher_logits) % 8 == 0) {
+      F.tsrc = TSRC_MEM_RING;
+    } else if (pl.tsrc == TSRC_MEM) {  // (rows the ring cannot read: 128-token tiles, the same ranges)
+      F.n_ttiles = (int)cdiv(pl.N, 128);
+      grid = F.n_ttiles * pl.n_vranges;
+    }
+  }
   const double scan_flops = 2.0 * (double)pl.N * (double)pl.V *
                             ((double)pl.H + ((pl.tsrc == TSRC_SHARED || pl.tsrc == TSRC_SEP) ? (double)pl.Ht : 0.0));
   { Timed tm_(ORDA_K_SCAN, s, scan_flops, scan_flops); ORDA_CHECK_LAUNCH(launch_scan<T>(F, grid, s)); }

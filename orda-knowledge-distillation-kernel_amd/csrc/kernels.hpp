@@ -1267,7 +1267,7 @@ __device__ __forceinline__ void acc_fence(const AccPair16TL<T>& p) {
 // (128 tokens, vocabulary range) mapping, partial output and logits store.
 template <class T, int SV, bool STORE, int TL = TL_NONE>
 __global__ __launch_bounds__(kThreads4, 1) void k_scan16(FusedParams P) {
-  static_assert(TL == TL_NONE || (!sv_phase1(SV) && STORE), "teacher logits from memory: one-pass, stored");
+  static_assert(TL == TL_NONE || STORE || TL != TL_FROM_L, "logits read back from L: stored");
   static_assert(TL != TL_STUDENT || SV == SV_STUDENT || SV == SV_STUDENT_T, "student-only tiles: no teacher");
   constexpr int NJ = TL ? 8 : 4;        // tokens per lane
   constexpr int kTok = TL ? 256 : 128;  // tokens per workgroup
@@ -1319,10 +1319,10 @@ __global__ __launch_bounds__(kThreads4, 1) void k_scan16(FusedParams P) {
     // a tile with tokens past N stores block by block
     const bool full = t0 + 256 <= P.N;
     if constexpr (TL == TL_STUDENT) {
-      if (full) store_tile16_staged<T>(c, P, x.v0, t0, 128, true, stage);
+      if (STORE && full) store_tile16_staged<T>(c, P, x.v0, t0, 128, true, stage);
       static_for<0, NJ>([&](auto J) {
         constexpr int j = decltype(J)::value;
-        if (!full) store_block16<T>(c, P, x.v0, t0, j);
+        if (STORE && !full) store_block16<T>(c, P, x.v0, t0, j);
         scan_variant<SV>(st[j], AccPair16S{c, j}, vlane0, vlimit, vlimit >= 256, lse_sT[j], lse_tT[j], P);
       });
     } else if constexpr (TL != TL_NONE) {
@@ -1332,16 +1332,16 @@ __global__ __launch_bounds__(kThreads4, 1) void k_scan16(FusedParams P) {
       uint2 raw[2][8];
       issue_teacher16<T, TL>(raw[0], P, x.v0, t0, 0);
       issue_teacher16<T, TL>(raw[1], P, x.v0, t0, 1);
-      if (full) store_tile16_staged<T>(c, P, x.v0, t0, 128, true, stage);
+      if (STORE && full) store_tile16_staged<T>(c, P, x.v0, t0, 128, true, stage);
       static_for<0, NJ>([&](auto J) {
         constexpr int j = decltype(J)::value;
         order_teacher16<T, TL>(raw[j & 1]);
-        if constexpr (TL == TL_FROM_MEM) {
+        if constexpr (TL == TL_FROM_MEM && STORE) {
           if (P.store_t) store_teacher16<T>(raw[j & 1], P, x.v0, t0, j);  // else the dlogits pass reads them in place
         }
         scan_variant<SV>(st[j], AccPair16TL<T>{c, j, raw[j & 1]}, vlane0, vlimit, vlimit >= 256, lse_sT[j],
                          lse_tT[j], P);
-        if (!full) store_block16<T>(c, P, x.v0, t0, j);
+        if (STORE && !full) store_block16<T>(c, P, x.v0, t0, j);
         if constexpr (j + 2 < NJ) issue_teacher16<T, TL>(raw[j & 1], P, x.v0, t0, j + 2);
       });
     } else {
@@ -2782,6 +2782,20 @@ inline bool scan_on_ring(const FusedParams& P) {
 #define ORDA_SCAN_CASE(T, SV)                                                                    \
   case SV:                                                                                       \
     if constexpr (sizeof(T) == 2) {                                                              \
+      if (P.tsrc == TSRC_NONE && P.student_ring) {                                               \
+        if constexpr (SV == SV_STUDENT || SV == SV_STUDENT_T)                                    \
+          hipLaunchKernelGGL((k_scan16<T, SV, false, TL_STUDENT>), dim3(grid), dim3(kThreads4), 0, s, P); \
+        else                                                                                     \
+          return hipErrorInvalidValue;                                                           \
+        break;                                                                                   \
+      }                                                                                          \
+      if (P.tsrc == TSRC_MEM_RING) {                                                             \
+        if constexpr (SV == SV_STUDENT || SV == SV_STUDENT_T || SV == SV_POW)                    \
+          return hipErrorInvalidValue;                                                           \
+        else                                                                                     \
+          hipLaunchKernelGGL((k_scan16<T, SV, false, TL_FROM_MEM>), dim3(grid), dim3(kThreads4), 0, s, P); \
+        break;                                                                                   \
+      }                                                                                          \
       if (scan_on_ring<T>(P)) {                                                                  \
         hipLaunchKernelGGL((k_scan16<T, SV, false>), dim3(grid), dim3(kThreads4), 0, s, P);      \
         break;                                                                                   \
@@ -2794,6 +2808,7 @@ inline bool scan_on_ring(const FusedParams& P) {
 
 #define ORDA_INSTANTIATE_SCAN(T)                                                     \
   template <> hipError_t launch_scan<T>(const FusedParams& P, int grid, hipStream_t s) { \
+    if (P.tsrc == TSRC_MEM_RING && (P.V % 4 != 0 || P.H <= 64)) return hipErrorInvalidValue; \
     switch (scan_variant_of(P)) {                                                    \
       ORDA_SCAN_CASE(T, SV_STUDENT)                                                  \
       ORDA_SCAN_CASE(T, SV_STUDENT_T)                                                \
