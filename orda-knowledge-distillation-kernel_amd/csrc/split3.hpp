@@ -5,7 +5,9 @@
 // remainder rounded to nearest, x3 exact), and a product a b is taken as the
 // six partial products a1 b1, a1 b2, a2 b1, a2 b2, a1 b3, a3 b1, exact in
 // the fp32 accumulators of v_mfma_f32_16x16x32_bf16; the three left out are
-// below 2^-24 |a b| (typically 2^-27, of either sign).  An MFMA sums 32 k at
+// below 2^-24 |a b| (typically 2^-27, of either sign).  An infinite operand
+// gives NaN products (inf - inf in its remainder), also where fp32 units would
+// give an infinity.  An MFMA sums 32 k at
 // once where the native fp32 MFMA sums 2, so a dot product rounds fewer times
 // than it does there.  Six bf16 products per fp32 one: 2500 / 6 = 417
 // TFLOP/s against the fp32 units' 157.  Measured against the native fp32
