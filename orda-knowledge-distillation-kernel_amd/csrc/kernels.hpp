@@ -164,12 +164,17 @@ struct AccPair4 {  // ring engine, the lane's token j: acc[mb][j] student, acc[m
 template <class AP>
 __device__ __forceinline__ void acc_fence(const AP&) {}
 
-// Accessors whose lane may hold teacher logits that are all -inf (a masked
-// stretch of the vocabulary) in one tile: 16 rows per lane instead of 64 or
-// 32.  The maxima they rescale by are then taken as 0 (exp(-inf) adds
-// nothing) instead of forming -inf - -inf.
+// Accessors whose teacher logits come from memory, where a caller may hold
+// -inf or its type's lowest value over a masked stretch of the vocabulary: a
+// lane's rows of its first tiles (16 to 64 rows within 64 to 128 of the
+// vocabulary) can all be masked.  The maxima they rescale by are then taken
+// as 0 (exp(-inf) adds nothing) instead of forming -inf - -inf, a NaN that the
+// next tile's finite maximum would carry into the row's sums.  kMaskedMax: a
+// maximum below it times log2(e) / T would overflow, so it counts as -inf.
+constexpr float kMaskedMax = -1e37f;
 template <class AP>
 struct GuardMasked : std::false_type {};
+template <> struct GuardMasked<AccPair2> : std::true_type {};
 
 // Phase 0: online softmax statistics of this lane's token over its
 // vocabulary rows of the tile (64 or 32, AP::Lay).  Template flags remove work that the problem
@@ -177,6 +182,10 @@ struct GuardMasked : std::false_type {};
 template <bool HAS_T, int FAM, bool T1, bool MASK, class AP, int NPOW = 3>
 __device__ __forceinline__ void scan_tile(RowState& S, const AP& acc, int vlane0, int64_t vlimit,
                                           const FusedParams& P) {
+  // (the two-stage lanes' three power sums spill as it is, and multiply an
+  // infinite logit by 0 anyway)
+  constexpr bool kGuard =
+      GuardMasked<AP>::value && !(std::is_same<AP, AccPair2>::value && FAM == FAM_POW && NPOW > 1);
   const float invT = P.invT;
   float tms = -kInf, tmt = -kInf, tmu0 = -kInf, tmu1 = -kInf, tmu2 = -kInf;
 #pragma unroll
@@ -213,7 +222,7 @@ __device__ __forceinline__ void scan_tile(RowState& S, const AP& acc, int vlane0
   float nmt = 0.f;
   if (HAS_T) {
     nmt = fmaxf(S.mt, tmt);
-    const bool none = GuardMasked<AP>::value && nmt == -kInf;  // every teacher logit so far is -inf
+    const bool none = kGuard && nmt < kMaskedMax;  // every teacher logit so far is masked
     const float d = none ? 0.f : S.mt - nmt;
     const float ct = fexp(d);
     const float ctT = T1 ? ct : fexp(d * invT);
@@ -224,16 +233,16 @@ __device__ __forceinline__ void scan_tile(RowState& S, const AP& acc, int vlane0
     }
     S.st *= ct;
     if (!T1) S.stt *= ctT;
-    S.mt = nmt;
+    S.mt = none ? -kInf : nmt;
     if (none) nmt = 0.f;
   }
   float nmu0 = 0.f, nmu1 = 0.f, nmu2 = 0.f;
   if (FAM == FAM_POW) {
     auto to_max = [&](float& m, float& sum, float tile_max) __attribute__((always_inline)) {
       const float nm = fmaxf(m, tile_max);
-      const bool none = GuardMasked<AP>::value && nm == -kInf;
+      const bool none = kGuard && nm < kMaskedMax;
       sum *= none ? 1.f : fexp(m - nm);
-      m = nm;
+      m = none ? -kInf : nm;
       return none ? 0.f : nm;
     };
     nmu0 = to_max(S.x[0], S.x[1], tmu0 * invT);
@@ -823,6 +832,7 @@ struct AccPairTL {  // student from accumulator block nb, teacher from ordered r
     return (r & 1) ? hi16<T>(w) : lo16<T>(w);
   }
 };
+template <class T> struct GuardMasked<AccPairTL<T>> : std::true_type {};
 template <class T>
 __device__ __forceinline__ void acc_fence(const AccPairTL<T>& p) {
   uint2* r = const_cast<uint2*>(p.tr);
@@ -1256,6 +1266,7 @@ struct AccPair16TL {  // student from block j, teacher from ordered raw register
     return (r & 1) ? hi16<T>(w) : lo16<T>(w);
   }
 };
+template <class T> struct GuardMasked<AccPair16TL<T>> : std::true_type {};
 template <class T>
 __device__ __forceinline__ void acc_fence(const AccPair16TL<T>& p) {
   uint2* r = const_cast<uint2*>(p.tr);
