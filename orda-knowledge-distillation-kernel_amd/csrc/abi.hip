@@ -189,13 +189,10 @@ inline int64_t splits_by_cost(bool f32, int64_t n, int64_t cols, int64_t K) {
 }
 
 // Least splits of K rows of `row_bytes` whose K ranges stay inside one 32-bit
-// buffer resource (the ring engine's MN-major operands).
-inline int splits_needed(int64_t row_bytes, int64_t K, int64_t& need) {
+// buffer resource (the ring engine's MN-major operands); past 64 none does.
+inline int64_t splits_needed(int64_t row_bytes, int64_t K) {
   const int64_t kmax = kRsrcBytes / row_bytes / 64 * 64;
-  if (kmax < 64) return fail(ORDA_EINVAL, "vocab rows of %lld bytes exceed a buffer resource", (long long)row_bytes);
-  need = cdiv(K, kmax);
-  if (need > 64) return fail(ORDA_EINVAL, "grad hidden needs %lld splits of the vocabulary (at most 64)", (long long)need);
-  return ORDA_OK;
+  return kmax < 64 ? 65 : cdiv(K, kmax);
 }
 
 int make_plan(const orda_problem_t* p, Plan& pl) {
@@ -375,17 +372,19 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
   if (pl.Vc < 256) pl.Vc = 256;
   if (pl.Vc > Vmax) pl.Vc = Vmax;
   pl.nchunks = cdiv(pl.V, pl.Vc);
-  auto bwd_split = [&](int64_t cols, int& splits, int64_t& kps) -> int {
+  // grad hidden's splits, where the two-phase backward computes one.  16-bit:
+  // K ranges inside one buffer resource as far as 64 splits reach (launch_gemm2
+  // takes its general kernel past that); the fp32 engine moves a 64-bit base.
+  pl.fused = (f & ORDA_GRADS_IN_FORWARD) != 0;
+  auto bwd_split = [&](int64_t cols, int& splits, int64_t& kps) {
     int64_t sp = splits_by_cost(f32, pl.N, cols, std::min(pl.Vc, pl.V));
-    int64_t need = 1;
-    ORDA_TRY_PLAN(splits_needed(std::max(pl.ldT, cols) * pl.eb, pl.Vc, need));
-    if (sp < need) sp = need;
+    const int64_t need = f32 ? 1 : splits_needed(std::max(pl.ldT, cols) * pl.eb, pl.Vc);
+    if (sp < need && need <= 64) sp = need;
     kps = round_up(cdiv(pl.Vc, sp), 64);
     splits = (int)cdiv(pl.Vc, kps);
-    return ORDA_OK;
   };
-  ORDA_TRY_PLAN(bwd_split(pl.H, pl.bwd_splits_s, pl.bwd_kps_s));
-  ORDA_TRY_PLAN(bwd_split(pl.Ht > 0 ? pl.Ht : pl.H, pl.bwd_splits_t, pl.bwd_kps_t));
+  if (!pl.fused && pl.need_gs) bwd_split(pl.H, pl.bwd_splits_s, pl.bwd_kps_s);
+  if (!pl.fused && pl.w_dln_t) bwd_split(pl.Ht, pl.bwd_splits_t, pl.bwd_kps_t);
   off = 0;
   pl.off_hT = (pl.need_gw && !f32) ? carve(off, (size_t)pl.H * pl.ldh * pl.eb) : 0;
   pl.off_htT = (sep && pl.w_dlt_t && !f32) ? carve(off, (size_t)pl.Ht * pl.NP * pl.eb) : 0;
@@ -397,7 +396,6 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
   pl.bwd_bytes = off + kAlign;
 
   // gradients inside forward: one token chunk of logits at a time
-  pl.fused = (f & ORDA_GRADS_IN_FORWARD) != 0;
   if (pl.fused) {
     // precomputed teachers: no teacher gradient; their logits (memory or the
     // frozen teacher GEMM) are stored next to the student's like a tied
@@ -517,8 +515,10 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
         }
       }
       // (the chunk's dlogits, ld = fldL, and the weight, ld = cols)
-      int64_t need = 1;
-      ORDA_TRY_PLAN(splits_needed(std::max<int64_t>(pl.fldL, cols) * pl.eb, pl.V, need));
+      const int64_t need = splits_needed(std::max<int64_t>(pl.fldL, cols) * pl.eb, pl.V);
+      if (need > 64)
+        return fail(ORDA_EINVAL, "grad hidden needs more than 64 splits of the vocabulary (rows of %lld bytes)",
+                    (long long)(std::max<int64_t>(pl.fldL, cols) * pl.eb));
       if (sp < need) sp = need;
       kps = round_up(cdiv(pl.V, sp), 64);
       splits = (int)cdiv(pl.V, kps);

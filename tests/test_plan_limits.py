@@ -1,0 +1,40 @@
+"""Plans at the ends of the stated sizes (CPU, through the library's planning
+entries): n_rows and vocab up to 2^30, hidden up to 2^22."""
+from __future__ import annotations
+
+import pytest
+
+from orda_ce_kernel import _native
+
+BF16, F16, F32 = 0, 1, 2
+
+
+def _problem(mode="tied", dtype=BF16, N=512, H=256, V=4096, Ht=None, flags=(), logits_dtype=None, div=0):
+    p = _native.Problem()
+    p.abi_version = _native.ABI_VERSION
+    p.mode, p.dtype, p.logits_dtype = _native.MODE[mode], dtype, dtype if logits_dtype is None else logits_dtype
+    p.n_rows, p.vocab, p.hidden, p.teacher_hidden = N, V, H, H if Ht is None else Ht
+    p.ignore_index = -100
+    for name in flags:
+        p.flags |= _native.FLAG[name]
+    p.divergence = div
+    p.temperature, p.student_ce_weight, p.teacher_ce_weight, p.kl_weight = 2.0, 1.0, 1.0, 1.0
+    return p
+
+
+GRADS = ("need_grad_student_hidden", "need_grad_weight", "compute_teacher_ce", "compute_divergence")
+
+
+@pytest.mark.parametrize("dtype,N,H,V,flags", [
+    (BF16, 1 << 23, 64, 4096, GRADS + ("grads_in_forward",)), (F32, 1 << 22, 64, 4096, GRADS + ("grads_in_forward",)),
+    (BF16, (1 << 24) + 64, 64, 4096, ("compute_divergence",)), (F32, (1 << 23) + 64, 64, 4096, ("compute_divergence",)),
+    (BF16, 1 << 30, 64, 4096, ()), (BF16, 64, 131072, 600000, ("compute_divergence",)),
+    (BF16, 64, 131072, 600000, GRADS), (F32, 64, 131072, 600000, GRADS), (F16, (1 << 24) + 64, 64, 4096, GRADS),
+    (BF16, 64, 131072, 600000, ("need_grad_weight",))])
+def test_large_calls_are_planned(dtype, N, H, V, flags):
+    """A limit of the grad-hidden GEMM's split ranges does not refuse calls that
+    run without that GEMM, nor two-phase ones, whose general kernel has none."""
+    p = _problem(dtype=dtype, N=N, H=H, V=V, flags=flags)
+    assert _native.forward_workspace_bytes(p) > 0
+    assert _native.saved_bytes(p) > 0
+    assert "grads_in_forward" in flags or _native.backward_workspace_bytes(p) > 0
