@@ -167,18 +167,20 @@ inline int rule_chunk_scale(const Plan& pl, const orda_problem_t* p, int64_t nco
 // 4 TB/s.  A small problem's few tiles spread over more CUs than at most 16
 // splits gave it (256 tokens, hidden 1024, vocabulary 32000, 4 tiles: 54 -> 35
 // us; 995 tokens, hidden 384, vocabulary 72448: 219 -> 105).
+// The search is part of every plan, several of a call: integer rounds, an end
+// where the partials alone cost more (256 tokens, hidden 1024, vocabulary
+// 32000: 1.3 -> 0.7 us a plan).
 inline int64_t splits_by_cost(bool f32, int64_t n, int64_t cols, int64_t K) {
   int64_t sp = 1;
   double best = 1e30;
-  const double tiles = (double)(cdiv(n, 256) * cdiv(cols, 256));
-  for (int c = 1; c <= 64 && (c == 1 || K / c >= (f32 ? 256 : 512)); ++c) {
+  const int64_t tiles = cdiv(n, 256) * cdiv(cols, 256);
+  const double part = (double)(n * cols) * 8.0 / 4e6;  // one split's partial
+  for (int64_t c = 1; c <= 64 && (c == 1 || (K / c >= (f32 ? 256 : 512) && part * c < best)); ++c) {
     double cost;
     if (f32) {
-      cost = std::min(s3_cost(n, cols, K, c, true), s3_cost(n, cols, K, c, false));
+      cost = std::min(s3_cost(n, cols, K, (int)c, true), s3_cost(n, cols, K, (int)c, false));
     } else {
-      const double rounds = std::ceil(tiles * (double)c / (double)kPersistentGroups);
-      cost = rounds * (std::ceil((double)K / (double)c / 64.0) * 1.4 + 10.0) +
-             (c > 1 ? (double)(c * n * cols) * 8.0 / 4e6 : 0.0);
+      cost = (double)cdiv(tiles * c, kPersistentGroups) * ((double)cdiv(K, 64 * c) * 1.4 + 10.0) + (c > 1 ? part * c : 0.0);
     }
     if (cost < best) {
       best = cost;
@@ -526,7 +528,9 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
     };
     auto both_splits = [&](bool fine) -> int {
       ORDA_TRY_PLAN(split_plan(pl.H, fine, pl.splits_s, pl.kps_s));
-      return split_plan(pl.Ht, fine, pl.splits_t, pl.kps_t);
+      pl.splits_t = pl.splits_s;
+      pl.kps_t = pl.kps_s;
+      return pl.Ht == pl.H || pl.Ht <= 0 ? ORDA_OK : split_plan(pl.Ht, fine, pl.splits_t, pl.kps_t);
     };
     ORDA_TRY_PLAN(both_splits(true));
     pl.f8 = (p->flags & ORDA_FP8_LOGITS) != 0;

@@ -38,3 +38,13 @@ def test_large_calls_are_planned(dtype, N, H, V, flags):
     assert _native.forward_workspace_bytes(p) > 0
     assert _native.saved_bytes(p) > 0
     assert "grads_in_forward" in flags or _native.backward_workspace_bytes(p) > 0
+
+
+@pytest.mark.parametrize("dtype", [BF16, F32])
+def test_cached_logits_need_no_teacher_hidden_size(dtype):
+    """Teacher logits come without a hidden size; also a plan past the static
+    scratch, which is planned again with fewer splits, divides by none."""
+    p = _problem("precomputed_logits", dtype, N=1024, H=512, V=60000, Ht=0,
+                 flags=("need_grad_student_hidden", "need_grad_weight", "compute_divergence", "grads_in_forward"))
+    assert _native.forward_workspace_bytes(p) > 64 << 20
+    assert _native.plan_info(p)["grad_hidden_splits"] >= 1
