@@ -391,7 +391,9 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
   pl.off_hT = (pl.need_gw && !f32) ? carve(off, (size_t)pl.H * pl.ldh * pl.eb) : 0;
   pl.off_htT = (sep && pl.w_dlt_t && !f32) ? carve(off, (size_t)pl.Ht * pl.NP * pl.eb) : 0;
   pl.off_dLT = (pl.bwd_student || pl.bwd_teacher) ? carve(off, (size_t)pl.Vc * pl.ldT * pl.eb) : 0;
-  const int64_t part_s = pl.need_gs ? pl.bwd_splits_s * pl.H : 0, part_t = pl.w_dln_t ? pl.bwd_splits_t * pl.Ht : 0;
+  // (one split: stored at once, or added up over the chunks in place)
+  const int64_t part_s = pl.need_gs && pl.bwd_splits_s > 1 ? pl.bwd_splits_s * pl.H : 0;
+  const int64_t part_t = pl.w_dln_t && pl.bwd_splits_t > 1 ? pl.bwd_splits_t * pl.Ht : 0;
   pl.off_bsplit = carve(off, (size_t)std::max(part_s, part_t) * pl.N * 4);
   pl.off_g32s = (pl.need_gs && pl.nchunks > 1) ? carve(off, (size_t)pl.N * pl.H * 4) : 0;
   pl.off_g32t = (pl.w_dln_t && pl.nchunks > 1) ? carve(off, (size_t)pl.N * pl.Ht * 4) : 0;
@@ -917,7 +919,9 @@ int run_backward(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* 
                       both ? 2 * NP : NP));
     if (sep && pl.need_gwt && pl.w_dlt_t)
       ORDA_TRY(grad_w(dLT + NP * eb, t->teacher_hidden, nullptr, htT, NP, Ht, t->grad_teacher_weight, NP));
-    // grad hidden (+)= dL W
+    // grad hidden (+)= dL W.  One split: rounded as it is stored where there is
+    // one chunk, else summed in g32 by the GEMMs (32768 tokens, hidden 5120: no
+    // 640 MiB of partials beside it) and rounded after the last.
     const int gmode = pl.nchunks == 1 ? GEMM_STORE
                       : c == 0 ? GEMM_ACC_FIRST
                       : c == pl.nchunks - 1 ? GEMM_ACC_LAST : GEMM_ACC;
@@ -925,14 +929,21 @@ int run_backward(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* 
                            int64_t kps) -> int {
       const double fl = 2.0 * (double)N * (double)cols * (double)vcc;
       const int sp = (int)std::min<int64_t>(splits, cdiv(vcc, kps));  // (a short last chunk has fewer)
+      const int mode = splits > 1 ? GEMM_SPLIT : pl.nchunks == 1 ? GEMM_STORE : c == 0 ? GEMM_SPLIT : GEMM_ACC;
+      void* C = mode == GEMM_STORE ? dst : nullptr;
+      float* C32 = mode == GEMM_STORE ? nullptr : splits > 1 ? bsplit : g32;
       if constexpr (sizeof(T) == 4)
-        ORDA_TRY(gemm_s3(MNMAJ, MNMAJ, A, pl.ldT, Wx, nullptr, cols, 0, vcc, 0, nullptr, bsplit, cols, N, cols, vcc,
-                         GEMM_SPLIT, sp, kps, s, ORDA_K_GEMM_H, fl));
+        ORDA_TRY(gemm_s3(MNMAJ, MNMAJ, A, pl.ldT, Wx, nullptr, cols, 0, vcc, 0, C, C32, cols, N, cols, vcc, mode, sp,
+                         kps, s, ORDA_K_GEMM_H, fl));
       else
-        ORDA_TRY(gemm2<T>(MNMAJ, MNMAJ, A, pl.ldT, Wx, cols, nullptr, 0, vcc, vcc, 0, nullptr, bsplit, cols, N, cols,
-                          vcc, GEMM_SPLIT, sp, kps, s, ORDA_K_GEMM_H, fl));
+        ORDA_TRY(gemm2<T>(MNMAJ, MNMAJ, A, pl.ldT, Wx, cols, nullptr, 0, vcc, vcc, 0, C, C32, cols, N, cols, vcc, mode,
+                          sp, kps, s, ORDA_K_GEMM_H, fl, mode == GEMM_STORE ? late : nullptr));
+      if (splits == 1 && (mode == GEMM_STORE || c + 1 < pl.nchunks)) return ORDA_OK;
       Timed tm_(ORDA_K_AUX, s, 0.0, 0.0);
-      ORDA_CHECK_LAUNCH(launch_splitk_reduce<T>(bsplit, sp, N * cols, dst, cols, N, cols, late, s, g32, gmode));
+      if (splits == 1)
+        ORDA_CHECK_LAUNCH(launch_splitk_reduce<T>(g32, 1, N * cols, dst, cols, N, cols, late, s));
+      else
+        ORDA_CHECK_LAUNCH(launch_splitk_reduce<T>(bsplit, sp, N * cols, dst, cols, N, cols, late, s, g32, gmode));
       return ORDA_OK;
     };
     if (pl.need_gs)

@@ -20,6 +20,8 @@ static hipError_t gemm_s3_go(const GemmParams& P, hipStream_t s) {
     hipLaunchKernelGGL((k_gemm_s3<C, MNMAJ, MNMAJ, GEMM_STORE>), g, b, 0, s, P);
   } else if (P.la == MNMAJ && P.mode == GEMM_SPLIT) {
     hipLaunchKernelGGL((k_gemm_s3<C, MNMAJ, MNMAJ, GEMM_SPLIT>), g, b, 0, s, P);
+  } else if (P.la == MNMAJ && P.mode == GEMM_ACC && P.splits == 1) {
+    hipLaunchKernelGGL((k_gemm_s3<C, MNMAJ, MNMAJ, GEMM_ACC>), g, b, 0, s, P);
   } else {
     return hipErrorInvalidValue;
   }

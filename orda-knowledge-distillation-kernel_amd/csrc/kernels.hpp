@@ -1860,7 +1860,7 @@ __global__ __launch_bounds__(kThreads4, 1) void k_gemm4(GemmParams P) {
     const int rl = lane & 15;          // C row of the lane within a block
     const int cq = 4 * (lane >> 4);    // first of the lane's 4 columns within a block (before the trade)
     const int cg = g8(lane);           // first of the lane's 8 columns within a block pair (after the trade)
-    if constexpr (MODE == GEMM_SPLIT) {
+    if constexpr (MODE == GEMM_SPLIT || MODE == GEMM_ACC) {
       float* D = P.C32 + (int64_t)x.split * P.split_stride + (int64_t)x.m0 * ldc + x.n0;
       if (mlim == 256 && nlim == 256) {
 #pragma unroll
@@ -1871,9 +1871,15 @@ __global__ __launch_bounds__(kThreads4, 1) void k_gemm4(GemmParams P) {
             const int nb = (pr >> 1) * 4 + (pr & 1) * 2;  // block pairs (0,1) (2,3) (4,5) (6,7)
             float xv[4], yv[4];
             trade16(c[mb][nb], c[mb][nb + 1], xv, yv);
-            float* p = rp + col16(nb, wn) + cg;
-            *reinterpret_cast<float4*>(p) = make_float4(xv[0], xv[1], xv[2], xv[3]);
-            *reinterpret_cast<float4*>(p + 4) = make_float4(yv[0], yv[1], yv[2], yv[3]);
+            float4* p = reinterpret_cast<float4*>(rp + col16(nb, wn) + cg);
+            float4 u = make_float4(xv[0], xv[1], xv[2], xv[3]), v = make_float4(yv[0], yv[1], yv[2], yv[3]);
+            if constexpr (MODE == GEMM_ACC) {
+              const float4 a = p[0], b = p[1];
+              u = make_float4(u.x + a.x, u.y + a.y, u.z + a.z, u.w + a.w);
+              v = make_float4(v.x + b.x, v.y + b.y, v.z + b.z, v.w + b.w);
+            }
+            p[0] = u;
+            p[1] = v;
             __builtin_amdgcn_sched_barrier(0);
           }
         }
@@ -1888,7 +1894,10 @@ __global__ __launch_bounds__(kThreads4, 1) void k_gemm4(GemmParams P) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const float v = acc16_get(c[mb][nb], e);
-            if (mm < mlim && cc + e < nlim) D[(int64_t)mm * ldc + cc + e] = v;
+            if (mm < mlim && cc + e < nlim) {
+              float* p = D + (int64_t)mm * ldc + cc + e;
+              *p = MODE == GEMM_ACC ? *p + v : v;
+            }
           }
         }
       }
@@ -3301,7 +3310,7 @@ inline void gemm2_go(const GemmParams& P, hipStream_t s) {
       return;
     }
   }
-  if constexpr (sizeof(T) == 2 && LA == MNMAJ && LB == MNMAJ && (MODE == GEMM_STORE || MODE == GEMM_SPLIT)) {
+  if constexpr (sizeof(T) == 2 && LA == MNMAJ && LB == MNMAJ) {
     const int64_t lim = 0x7fffffffll / (int64_t)sizeof(T);
     if (P.k_per_split > 64 && P.k_per_split * P.lda < lim && P.k_per_split * P.ldb < lim) {
       hipLaunchKernelGGL((k_gemm4<T, MNMAJ, MNMAJ, MODE>), dim3(grid), dim3(kThreads4), 0, s, P);
@@ -3318,6 +3327,7 @@ inline void gemm2_go(const GemmParams& P, hipStream_t s) {
       case KMAJ * 100 + MNMAJ * 10 + GEMM_ACC_T: gemm2_go<T, KMAJ, MNMAJ, GEMM_ACC_T>(P, s); break; \
       case MNMAJ * 100 + MNMAJ * 10 + GEMM_STORE: gemm2_go<T, MNMAJ, MNMAJ, GEMM_STORE>(P, s); break; \
       case MNMAJ * 100 + MNMAJ * 10 + GEMM_SPLIT: gemm2_go<T, MNMAJ, MNMAJ, GEMM_SPLIT>(P, s); break; \
+      case MNMAJ * 100 + MNMAJ * 10 + GEMM_ACC: gemm2_go<T, MNMAJ, MNMAJ, GEMM_ACC>(P, s); break; \
       case KMAJ * 100 + KMAJ * 10 + GEMM_STORE: gemm2_go<T, KMAJ, KMAJ, GEMM_STORE>(P, s); break; \
       case KMAJ * 100 + KMAJ * 10 + GEMM_ACC_T: gemm2_go<T, KMAJ, KMAJ, GEMM_ACC_T>(P, s); break; \
       case MNMAJ * 100 + KMAJ * 10 + GEMM_STORE: gemm2_go<T, MNMAJ, KMAJ, GEMM_STORE>(P, s); break; \

@@ -226,7 +226,7 @@ __device__ __forceinline__ void s3_loop(char* lds, int total, const Fetch& fetch
 
 // ------------------------------------------------------------------- GEMM
 // C[M x N] (GEMM_STORE, GEMM_ACC_T: C +=, GEMM_SPLIT: split s's K range
-// [s k_per_split, ...) to C32 + s split_stride) A B^T, fp32.  A K-major or
+// [s k_per_split, ...) to C32 + s split_stride, GEMM_ACC: C32 +=) A B^T, fp32.  A K-major or
 // MN-major; B K-major (one segment), or MN-major, for a K-major A in up to two
 // K segments as k_gemm2 (rows [0, b_kseg) from B, the first b_kval0 valid, the
 // rest from B1).  Persistent: workgroup b (in XCD order) runs work items b, b +
@@ -301,7 +301,7 @@ __global__ __launch_bounds__(C::kThreads, C::MB == 4 ? 2 : 3) void k_gemm_s3(Gem
     const Tile x = tile_of(mi++);
     const int ol = opaque_lane();
     const int mlim = (int)min<int64_t>(P.M - x.m0, RA), nlim = (int)min<int64_t>(P.N - x.n0, RB);
-    float* D = (MODE == GEMM_SPLIT ? P.C32 + x.split * P.split_stride : static_cast<float*>(P.C)) + x.m0 * P.ldc + x.n0;
+    float* D = (MODE == GEMM_SPLIT || MODE == GEMM_ACC ? P.C32 + x.split * P.split_stride : static_cast<float*>(P.C)) + x.m0 * P.ldc + x.n0;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
       const int m = wm * 16 * MB + mb * 16 + (ol & 15);
@@ -311,7 +311,7 @@ __global__ __launch_bounds__(C::kThreads, C::MB == 4 ? 2 : 3) void k_gemm_s3(Gem
         if (m < mlim && n < nlim) {
           float4* p = reinterpret_cast<float4*>(D + (int64_t)m * P.ldc + n);
           float4 o = make_float4(acc[mb][nb][0], acc[mb][nb][1], acc[mb][nb][2], acc[mb][nb][3]);
-          if constexpr (MODE == GEMM_ACC_T) {
+          if constexpr (MODE == GEMM_ACC_T || MODE == GEMM_ACC) {
             const float4 c = *p;
             o = make_float4(c.x + o.x, c.y + o.y, c.z + o.z, c.w + o.w);
           }

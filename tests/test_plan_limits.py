@@ -48,3 +48,12 @@ def test_cached_logits_need_no_teacher_hidden_size(dtype):
                  flags=("need_grad_student_hidden", "need_grad_weight", "compute_divergence", "grads_in_forward"))
     assert _native.forward_workspace_bytes(p) > 64 << 20
     assert _native.plan_info(p)["grad_hidden_splits"] >= 1
+
+
+@pytest.mark.parametrize("N,H,V", [(32768, 5120, 152064), (8192, 4096, 128256)])
+def test_two_phase_workspace_holds_one_fp32_sum(N, H, V):
+    """A grad-hidden GEMM of one split needs one fp32 [N x H] sum over the
+    vocabulary chunks beside the transposed rows and 512 MiB of dlogits."""
+    p = _problem(N=N, H=H, V=V, flags=GRADS)
+    got = _native.backward_workspace_bytes(p)
+    assert got <= 4 * N * H + 2 * 2 * N * H + (512 << 20) + (1 << 20), got / 2 ** 20
