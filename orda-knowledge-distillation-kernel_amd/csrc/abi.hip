@@ -744,14 +744,13 @@ int run_forward(const Plan& pl, const orda_problem_t* p, const orda_tensors_t* t
 }
 
 template <class T>
-int gemm(const void* A, int64_t lda, const void* B, int64_t ldb, void* C, float* C32, int64_t ldc, int64_t M,
-         int64_t N, int64_t K, int mode, hipStream_t s, int kind = ORDA_K_AUX, double alg = 0.0) {
+int gemm_abt(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, hipStream_t s) {
   GemmParams G{};
-  G.A = A; G.B = B; G.C = C; G.C32 = C32;
-  G.M = M; G.N = N; G.K = K; G.lda = lda; G.ldb = ldb; G.ldc = ldc;
-  G.tiles_m = (int)cdiv(M, 256); G.tiles_n = (int)cdiv(N, 256); G.mode = mode;
+  G.A = A; G.B = B; G.C = C;
+  G.M = M; G.N = N; G.K = K; G.lda = K; G.ldb = K; G.ldc = N;
+  G.tiles_m = (int)cdiv(M, 256); G.tiles_n = (int)cdiv(N, 256); G.mode = GEMM_STORE;
   if ((int64_t)G.tiles_m * G.tiles_n > 0x7fffffffll) return fail(ORDA_EINVAL, "gemm grid too large");
-  Timed tm_(kind, s, alg, 2.0 * (double)M * (double)N * (double)K);
+  Timed tm_(ORDA_K_AUX, s, 0.0, 2.0 * (double)M * (double)N * (double)K);
   ORDA_CHECK_LAUNCH(launch_gemm<T>(G, s));
   return ORDA_OK;
 }
@@ -1538,9 +1537,9 @@ int orda_gemm_abt(int32_t dtype, int64_t M, int64_t N, int64_t K, const void* A,
   if (!aligned16(A) || !aligned16(B)) return fail(ORDA_EINVAL, "A and B must be 16-byte aligned");
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (dtype) {
-    case ORDA_BF16: return gemm<bf16>(A, K, B, K, C, nullptr, N, M, N, K, GEMM_STORE, s);
-    case ORDA_F16: return gemm<f16>(A, K, B, K, C, nullptr, N, M, N, K, GEMM_STORE, s);
-    default: return gemm<float>(A, K, B, K, C, nullptr, N, M, N, K, GEMM_STORE, s);
+    case ORDA_BF16: return gemm_abt<bf16>(A, B, C, M, N, K, s);
+    case ORDA_F16: return gemm_abt<f16>(A, B, C, M, N, K, s);
+    default: return gemm_abt<float>(A, B, C, M, N, K, s);
   }
 }
 
@@ -1579,6 +1578,15 @@ int orda_gemm(int32_t dtype, int32_t a_mn, int32_t b_mn, int64_t M, int64_t N, i
   const int la = a_mn ? MNMAJ : KMAJ, lb = b_mn ? MNMAJ : KMAJ;
   auto go = [&](auto tag) -> int {
     using T = decltype(tag);
+    if constexpr (sizeof(T) == 4) {
+      // the loss's fp32 engine where it has the layouts (it writes C in fours)
+      if (N % 4 == 0 && !(la == MNMAJ && lb == KMAJ) && (sp == 1 || la == MNMAJ)) {
+        ORDA_TRY(gemm_s3(la, lb, A, lda, B, nullptr, ldb, K, K, 0, C, part, sp > 1 ? N : ldc, M, N, K,
+                         sp > 1 ? GEMM_SPLIT : GEMM_STORE, sp, kps, s, ORDA_K_AUX, 0.0));
+        if (sp > 1) ORDA_CHECK_LAUNCH(launch_splitk_reduce<T>(part, sp, M * N, C, ldc, M, N, nullptr, s));
+        return ORDA_OK;
+      }
+    }
     if (sp == 1)
       return gemm2<T>(la, lb, A, lda, B, ldb, nullptr, 0, K, K, 0, C, nullptr, ldc, M, N, K, GEMM_STORE, 1, 0, s,
                       ORDA_K_AUX, 0.0);

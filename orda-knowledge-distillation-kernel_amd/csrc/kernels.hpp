@@ -1504,14 +1504,13 @@ __global__ __launch_bounds__(kThreads) void k_dl(FusedParams P) {
 }
 
 // -------------------------------------------------------------- plain GEMM
-template <class T, int MODE>
+template <class T>
 __device__ __forceinline__ void gemm_epilogue(const f32x16 (&acc)[4][2], const GemmParams& P, int64_t m0,
                                               int64_t n0) {
   const int lane = threadIdx.x & 63;
   const int wm = wave_m(), wn = wave_n();
   // 32-bit offsets inside the tile; the tile base stays 64-bit.
   T* C = static_cast<T*>(P.C) + m0 * P.ldc + n0;
-  float* C32 = P.C32 + m0 * P.ldc + n0;
   const int ldc = (int)P.ldc;
   const int mlim = (int)min<int64_t>(P.M - m0, 256), nlim = (int)min<int64_t>(P.N - n0, 256);
 #pragma unroll
@@ -1523,21 +1522,14 @@ __device__ __forceinline__ void gemm_epilogue(const f32x16 (&acc)[4][2], const G
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int m = mrow0 + (r >> 2) * 8 + (r & 3);
-        if (m < mlim && n < nlim) {
-          const int o = m * ldc + n;
-          const float a = acc[mb][nb][r];
-          if (MODE == GEMM_STORE) C[o] = from_f32<T>(a);
-          else if (MODE == GEMM_ACC_FIRST) C32[o] = a;
-          else if (MODE == GEMM_ACC) C32[o] += a;
-          else C[o] = from_f32<T>(C32[o] + a);
-        }
+        if (m < mlim && n < nlim) C[m * ldc + n] = from_f32<T>(acc[mb][nb][r]);
       }
     }
 }
 
-// C[M x N] (= or +=) A[M x K] * B[N x K]^T.  Epilogue modes: STORE writes C
-// in T; ACC_FIRST/ACC write the fp32 accumulator C32; ACC_LAST adds C32 and
-// writes C in T.  Tiles are visited in bands of 8 tile rows, XCD by XCD.
+// C[M x N] = A[M x K] * B[N x K]^T in T, any ldc and alignment of C (the
+// exported orda_gemm_abt).  Tiles are visited in bands of 8 tile rows, XCD by
+// XCD.
 template <class T>
 __global__ __launch_bounds__(kThreads) void k_gemm(GemmParams P) {
   __shared__ __attribute__((aligned(16))) char lds[kLdsBytes];
@@ -1556,12 +1548,7 @@ __global__ __launch_bounds__(kThreads) void k_gemm(GemmParams P) {
   zero_acc(acc);
   mainloop<T, true, true>(acc, lds, A + m0 * P.lda, P.lda, P.M - m0, B + n0 * P.ldb, P.ldb, P.N - n0,
                           B + (n0 + 128) * P.ldb, P.ldb, P.N - n0 - 128, P.K);
-  switch (P.mode) {
-    case GEMM_STORE: gemm_epilogue<T, GEMM_STORE>(acc, P, m0, n0); break;
-    case GEMM_ACC_FIRST: gemm_epilogue<T, GEMM_ACC_FIRST>(acc, P, m0, n0); break;
-    case GEMM_ACC: gemm_epilogue<T, GEMM_ACC>(acc, P, m0, n0); break;
-    default: gemm_epilogue<T, GEMM_ACC_LAST>(acc, P, m0, n0); break;
-  }
+  gemm_epilogue<T>(acc, P, m0, n0);
 }
 
 // ------------------------------------------------------------ general GEMM
@@ -1674,15 +1661,14 @@ __device__ __forceinline__ void gemm_epilogue_q(const f32x16 (&acc)[4][2], const
 #pragma unroll
             for (int e = 0; e < 4; ++e) c[e] = (c[e] + o[e]) * cs;
             store4(C + off, c, full, cnt);
-          } else if constexpr (MODE == GEMM_ACC_FIRST || MODE == GEMM_SPLIT) {
+          } else if constexpr (MODE == GEMM_SPLIT) {
             store4(D + off, o, full, cnt);
           } else {
             float c[4];
             load4(D + off, c, full, cnt);
 #pragma unroll
             for (int e = 0; e < 4; ++e) c[e] += o[e];
-            if constexpr (MODE == GEMM_ACC) store4(D + off, c, full, cnt);
-            else store4(C + off, c, full, cnt);
+            store4(D + off, c, full, cnt);
           }
         }
       }
@@ -3319,18 +3305,20 @@ inline void gemm2_go(const GemmParams& P, hipStream_t s) {
   }
   hipLaunchKernelGGL((k_gemm2<T, LA, LB, MODE>), dim3(grid), dim3(kThreads), 0, s, P);
 }
-#define ORDA_INSTANTIATE_GEMM2(T)                                                          \
-  template <> hipError_t launch_gemm2<T>(const GemmParams& P, hipStream_t s) {             \
-    const int key = P.la * 100 + P.lb * 10 + P.mode;                                       \
-    switch (key) {                                                                         \
-      case KMAJ * 100 + MNMAJ * 10 + GEMM_STORE: gemm2_go<T, KMAJ, MNMAJ, GEMM_STORE>(P, s); break; \
-      case KMAJ * 100 + MNMAJ * 10 + GEMM_ACC_T: gemm2_go<T, KMAJ, MNMAJ, GEMM_ACC_T>(P, s); break; \
-      case MNMAJ * 100 + MNMAJ * 10 + GEMM_STORE: gemm2_go<T, MNMAJ, MNMAJ, GEMM_STORE>(P, s); break; \
-      case MNMAJ * 100 + MNMAJ * 10 + GEMM_SPLIT: gemm2_go<T, MNMAJ, MNMAJ, GEMM_SPLIT>(P, s); break; \
-      case MNMAJ * 100 + MNMAJ * 10 + GEMM_ACC: gemm2_go<T, MNMAJ, MNMAJ, GEMM_ACC>(P, s); break; \
-      case KMAJ * 100 + KMAJ * 10 + GEMM_STORE: gemm2_go<T, KMAJ, KMAJ, GEMM_STORE>(P, s); break; \
-      case KMAJ * 100 + KMAJ * 10 + GEMM_ACC_T: gemm2_go<T, KMAJ, KMAJ, GEMM_ACC_T>(P, s); break; \
-      case MNMAJ * 100 + KMAJ * 10 + GEMM_STORE: gemm2_go<T, MNMAJ, KMAJ, GEMM_STORE>(P, s); break; \
+#define ORDA_GEMM2_CASE(LA, LB, MODE) \
+  case LA * 100 + LB * 10 + MODE: gemm2_go<T, LA, LB, MODE>(P, s); break;
+#define ORDA_INSTANTIATE_GEMM2(TYPE)                                                       \
+  template <> hipError_t launch_gemm2<TYPE>(const GemmParams& P, hipStream_t s) {          \
+    using T = TYPE;                                                                        \
+    switch (P.la * 100 + P.lb * 10 + P.mode) {                                             \
+      ORDA_GEMM2_CASE(KMAJ, MNMAJ, GEMM_STORE)                                             \
+      ORDA_GEMM2_CASE(KMAJ, MNMAJ, GEMM_ACC_T)                                             \
+      ORDA_GEMM2_CASE(MNMAJ, MNMAJ, GEMM_STORE)                                            \
+      ORDA_GEMM2_CASE(MNMAJ, MNMAJ, GEMM_SPLIT)                                            \
+      ORDA_GEMM2_CASE(MNMAJ, MNMAJ, GEMM_ACC)                                              \
+      ORDA_GEMM2_CASE(KMAJ, KMAJ, GEMM_STORE)                                              \
+      ORDA_GEMM2_CASE(KMAJ, KMAJ, GEMM_ACC_T)                                              \
+      ORDA_GEMM2_CASE(MNMAJ, KMAJ, GEMM_STORE)                                             \
       default: return hipErrorInvalidValue;                                                \
     }                                                                                      \
     return hipGetLastError();                                                              \

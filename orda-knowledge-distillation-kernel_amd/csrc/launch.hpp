@@ -22,10 +22,10 @@ enum TeacherSource {
                      // teacher columns (V a multiple of 4)
 };
 
-// GEMM epilogues: STORE writes C in T; ACC_FIRST / ACC / ACC_LAST build an
-// fp32 sum in C32 over calls (the last one writes C); ACC_T adds into C in
-// T (C = T(C + A B^T)); SPLIT writes split s's fp32 partial to
-// C32 + s * split_stride.
+// GEMM epilogues: STORE writes C in T; ACC_T adds into C in T (C = T(C + A
+// B^T)); ACC adds into C32; SPLIT writes split s's fp32 partial to C32 + s *
+// split_stride.  launch_splitk_reduce builds an fp32 sum over calls with
+// ACC_FIRST / ACC / ACC_LAST.
 enum GemmMode { GEMM_STORE = 0, GEMM_ACC_FIRST = 1, GEMM_ACC = 2, GEMM_ACC_LAST = 3, GEMM_ACC_T = 4, GEMM_SPLIT = 5 };
 
 struct FusedParams {
