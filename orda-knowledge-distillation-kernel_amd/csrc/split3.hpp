@@ -1,21 +1,27 @@
 // fp32 GEMMs and scans on the bf16 matrix cores of gfx950.
 //
 // An fp32 value is the exact sum of three bf16 values, x = x1 + x2 + x3 (8 +
-// 8 + 8 significant bits: x1 truncated, so that no finite x overflows, x2 the
-// remainder rounded to nearest, x3 exact), and a product a b is taken as the
-// six partial products a1 b1, a1 b2, a2 b1, a2 b2, a1 b3, a3 b1, exact in
-// the fp32 accumulators of v_mfma_f32_16x16x32_bf16; the three left out are
-// below 2^-24 |a b| (typically 2^-27, of either sign).  An infinite operand
-// gives NaN products (inf - inf in its remainder), also where fp32 units would
-// give an infinity.  An MFMA sums 32 k at
-// once where the native fp32 MFMA sums 2, so a dot product rounds fewer times
-// than it does there.  Six bf16 products per fp32 one: 2500 / 6 = 417
-// TFLOP/s against the fp32 units' 157.  Measured against the native fp32
-// MFMA (32x32x2) kernels this replaces: 170 against 110 TFLOP/s in the
+// 8 + 8 significant bits: x1 and x2 rounded to nearest, so |x2| <= 2^-8 |x| and
+// |x3| <= 2^-17 |x|, either sign; x3 exact above 2^-109, below it off by at most
+// 2^-133; |x| past the largest bf16 value keeps its excess in x2), and a product
+// a b is taken as the six partial products a1 b1, a1 b2, a2 b1, a2 b2, a1 b3,
+// a3 b1, exact in the fp32 accumulators of v_mfma_f32_16x16x32_bf16; the three
+// left out are below 2^-24 + 2^-34 of |a b|, of either sign.  The signs matter:
+// an MFMA drops bits of products far below its accumulator, and with x1
+// truncated (x2 of x's sign) a sum of 4096 positive products lost 3.6e-6 of its
+// value, 5.3e-7 with x1 rounded and 8.5e-7 on the native fp32 MFMA.  An infinite
+// operand gives NaN products (inf - inf in its remainder), also where fp32
+// units would give an infinity.  An MFMA sums 32 k at once where the native
+// fp32 MFMA sums 2, so a long dot product rounds fewer times than it does there:
+// error relative to the sum of |a b|, normal operands, K = 64, 1024, 4096:
+// 1.8e-8, 2.4e-8, 2.5e-8 against 2.8e-8.  Six bf16 products per fp32 one: 2500
+// / 6 = 417 TFLOP/s against the fp32 units' 157.  Measured against the native
+// fp32 MFMA (32x32x2) kernels this replaces: 170 against 110 TFLOP/s in the
 // GEMMs; 1000 tokens, hidden 1000, teacher hidden 1200, vocabulary 30001: 2.44
-// -> 1.48 ms a step, gradients off float64 by 6.4e-7 of their norm against
-// 9e-7; 512 x 256 x 4096: 504 -> 128 us of kernels.  The matrix cores are busy
-// 56% of the cycles at 1.94 GHz (the socket's power limit).
+// -> 1.50 ms a step, gradients off float64 by 6.4e-7 of their norm against
+// 9e-7; 512 x 256 x 4096: 504 -> 128 us of kernels.  All eight products down to
+// 2^-34 take 1.70 ms for the former at the same error.  The matrix cores are
+// busy 56% of the cycles at 1.94 GHz (the socket's power limit).
 //
 // Workgroup: WA x 2 waves, wave tile (16 MB) squared, K steps of 32.  An
 // operand's K step goes global -> registers (the step after next's loads are
@@ -68,12 +74,14 @@ __device__ __forceinline__ uint32_t s3_addr(int row, int chunk) {
 // at `d`, the row's s3_addr plus 8 (k quad % 2) in the operand's first plane.
 template <int PL>
 __device__ __forceinline__ void s3_put(char* d, float x0, float x1, float x2, float x3) {
-  const uint32_t a[4] = {__float_as_uint(x0), __float_as_uint(x1), __float_as_uint(x2), __float_as_uint(x3)};
+  constexpr float kMaxBf16 = 3.38953139e38f;
+  auto top = [](float x) { return __builtin_amdgcn_fmed3f(x, -kMaxBf16, kMaxBf16); };
   float r[4], q[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) r[i] = __uint_as_float(a[i]) - __uint_as_float(a[i] & 0xffff0000u);
-  const uint2 p1 = make_uint2(__builtin_amdgcn_perm(a[1], a[0], 0x07060302u),
-                              __builtin_amdgcn_perm(a[3], a[2], 0x07060302u));
+  const uint2 p1 = make_uint2(pack2<bf16>(top(x0), top(x1)), pack2<bf16>(top(x2), top(x3)));
+  r[0] = x0 - __uint_as_float(p1.x << 16);
+  r[1] = x1 - __uint_as_float(p1.x & 0xffff0000u);
+  r[2] = x2 - __uint_as_float(p1.y << 16);
+  r[3] = x3 - __uint_as_float(p1.y & 0xffff0000u);
   const uint2 p2 = make_uint2(pack2<bf16>(r[0], r[1]), pack2<bf16>(r[2], r[3]));
   q[0] = r[0] - __uint_as_float(p2.x << 16);
   q[1] = r[1] - __uint_as_float(p2.x & 0xffff0000u);
