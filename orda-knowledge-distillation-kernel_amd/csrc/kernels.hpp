@@ -175,6 +175,10 @@ constexpr float kMaskedMax = -1e37f;
 template <class AP>
 struct GuardMasked : std::false_type {};
 template <> struct GuardMasked<AccPair2> : std::true_type {};
+// The same for a lane's student logits: 16 rows per lane in fp32, whose logits
+// an infinite weight can mask.
+template <class AP>
+struct GuardStudent : std::false_type {};
 
 // Phase 0: online softmax statistics of this lane's token over its
 // vocabulary rows of the tile (64 or 32, AP::Lay).  Template flags remove work that the problem
@@ -205,19 +209,22 @@ __device__ __forceinline__ void scan_tile(RowState& S, const AP& acc, int vlane0
         }
       }
     }
-  if (MASK && tms == -kInf) return;  // no valid vocabulary row in this lane
+  constexpr bool kGuardS = GuardStudent<AP>::value;
+  if (MASK && (kGuardS ? vlane0 >= vlimit : tms == -kInf)) return;  // no valid vocabulary row in this lane
   acc_fence(acc);
 
   // rescale the running state to the new maxima
-  const float nms = fmaxf(S.ms, tms);
+  float nms = fmaxf(S.ms, tms);
   {
-    const float d = S.ms - nms;
+    const bool none = kGuardS && nms < kMaskedMax;
+    const float d = none ? 0.f : S.ms - nms;
     const float cs = fexp(d);
     const float csT = T1 ? cs : fexp(d * invT);
     S.ss *= cs;
     if (!T1) S.sst *= csT;
     if (FAM == FAM_LIN) S.x[1] *= csT;
-    S.ms = nms;
+    S.ms = none ? -kInf : nms;
+    if (none) nms = 0.f;
   }
   float nmt = 0.f;
   if (HAS_T) {

@@ -3,25 +3,32 @@
 // An fp32 value is the exact sum of three bf16 values, x = x1 + x2 + x3 (8 +
 // 8 + 8 significant bits: x1 and x2 rounded to nearest, so |x2| <= 2^-8 |x| and
 // |x3| <= 2^-17 |x|, either sign; x3 exact above 2^-109, below it off by at most
-// 2^-133; |x| past the largest bf16 value keeps its excess in x2), and a product
+// 2^-133), and a product
 // a b is taken as the six partial products a1 b1, a1 b2, a2 b1, a2 b2, a1 b3,
 // a3 b1, exact in the fp32 accumulators of v_mfma_f32_16x16x32_bf16; the three
 // left out are below 2^-24 + 2^-34 of |a b|, of either sign.  The signs matter:
 // an MFMA drops bits of products far below its accumulator, and with x1
 // truncated (x2 of x's sign) a sum of 4096 positive products lost 3.6e-6 of its
-// value, 5.3e-7 with x1 rounded and 8.5e-7 on the native fp32 MFMA.  An infinite
-// operand gives NaN products (inf - inf in its remainder), also where fp32
-// units would give an infinity.  An MFMA sums 32 k at once where the native
-// fp32 MFMA sums 2, so a long dot product rounds fewer times than it does there:
-// error relative to the sum of |a b|, normal operands, K = 64, 1024, 4096:
-// 1.8e-8, 2.4e-8, 2.5e-8 against 2.8e-8.  Six bf16 products per fp32 one: 2500
-// / 6 = 417 TFLOP/s against the fp32 units' 157.  Measured against the native
-// fp32 MFMA (32x32x2) kernels this replaces: 170 against 110 TFLOP/s in the
-// GEMMs; 1000 tokens, hidden 1000, teacher hidden 1200, vocabulary 30001: 2.44
-// -> 1.50 ms a step, gradients off float64 by 6.4e-7 of their norm against
-// 9e-7; 512 x 256 x 4096: 504 -> 128 us of kernels.  All eight products down to
-// 2^-34 take 1.70 ms for the former at the same error.  The matrix cores are
-// busy 56% of the cycles at 1.94 GHz (the socket's power limit).
+// value, 5.3e-7 with x1 rounded and 8.5e-7 on the native fp32 MFMA.  An MFMA
+// sums 32 k at once where the native fp32 MFMA sums 2, so a long dot product
+// rounds fewer times than it does there: error relative to the sum of |a b|,
+// normal operands, K = 64, 1024, 4096: 1.8e-8, 2.4e-8, 2.5e-8 against 2.8e-8.
+// Six bf16 products per fp32 one: 2500 / 6 = 417 TFLOP/s against the fp32
+// units' 157.  Measured against the native fp32 MFMA (32x32x2) kernels this
+// replaces: 170 against 110 TFLOP/s in the GEMMs; 1000 tokens, hidden 1000,
+// teacher hidden 1200, vocabulary 30001: 2.44 -> 1.50 ms a step, gradients off
+// float64 by 6.4e-7 of their norm against 9e-7; 512 x 256 x 4096: 504 -> 128 us
+// of kernels.  All eight products down to 2^-34 take 1.70 ms for the former at
+// the same error.  The matrix cores are busy 56% of the cycles at 1.94 GHz (the
+// socket's power limit).
+//
+// Operands without such a split (infinities, values that round past the bf16
+// range) and sums of at most 16 products, where six roundings are more than the
+// sum's own (one product: 3.4e-8 of it against 2.5e-8): the tile is done over on
+// the native fp32 MFMA before it is written out.  The loaders keep the largest
+// magnitude they split (under 1% of the first call above); looking at it in
+// every K step took 7% of that call and multiplying single steps natively there
+// 9% (loads issued later, registers).
 //
 // Workgroup: WA x 2 waves, wave tile (16 MB) squared, K steps of 32.  An
 // operand's K step goes global -> registers (the step after next's loads are
@@ -59,7 +66,7 @@ struct S3Cfg {
   static constexpr int kThreads = WA * 128;
   static constexpr int kRowsA = 16 * MB * WA, kRowsB = 32 * MB;
   static constexpr int kStage = (kRowsA + kRowsB) * 192;  // three planes of 64 bytes per row
-  static constexpr int kLds = 2 * kStage;
+  static constexpr int kLds = 2 * kStage + 16;  // and the marks
 };
 using S3Big = S3Cfg<4, 4>;
 using S3Small = S3Cfg<2, 2>;
@@ -70,14 +77,16 @@ __device__ __forceinline__ uint32_t s3_addr(int row, int chunk) {
   return (uint32_t)((row >> 2) * 256 + (((row & 3) ^ x) << 6) + ((chunk ^ f ^ (((row >> 4) & 1) << 1)) << 4));
 }
 
+// Largest magnitude that rounds to a finite bf16 value (0x7f7f7fff).
+constexpr float kS3Max = 3.39617746e38f;
+constexpr int kS3Short = 16;  // sums of at most this many products are native
+
 // Four k values of one row to its three planes (8 bytes each, PL bytes apart)
 // at `d`, the row's s3_addr plus 8 (k quad % 2) in the operand's first plane.
 template <int PL>
 __device__ __forceinline__ void s3_put(char* d, float x0, float x1, float x2, float x3) {
-  constexpr float kMaxBf16 = 3.38953139e38f;
-  auto top = [](float x) { return __builtin_amdgcn_fmed3f(x, -kMaxBf16, kMaxBf16); };
   float r[4], q[4];
-  const uint2 p1 = make_uint2(pack2<bf16>(top(x0), top(x1)), pack2<bf16>(top(x2), top(x3)));
+  const uint2 p1 = make_uint2(pack2<bf16>(x0, x1), pack2<bf16>(x2, x3));
   r[0] = x0 - __uint_as_float(p1.x << 16);
   r[1] = x1 - __uint_as_float(p1.x & 0xffff0000u);
   r[2] = x2 - __uint_as_float(p1.y << 16);
@@ -100,6 +109,12 @@ __device__ __forceinline__ float4 s3_load(__amdgpu_buffer_rsrc_t rs, uint32_t of
   return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
 }
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t s3_rsrc(const float* p) { return uniform_rsrc(p, 0x7fffffff); }
+
+// (a NaN counts as nothing: its products are NaN on any path)
+__device__ __forceinline__ float s3_largest(float m, const float4& x) {
+  m = fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), m);
+  return fmaxf(fmaxf(fabsf(x.z), fabsf(x.w)), m);
+}
 
 // K-contiguous operand of R rows (NT threads): piece i of a thread is row
 // NT / 8 i + tid / 8, k 4 (tid % 8) .. + 3.  Rows past `rows` and k past
@@ -128,6 +143,11 @@ struct S3K {
 #pragma unroll
     for (int i = 0; i < NP; ++i) s3_put<R * 64>(d + i * kStride * 64, v[i].x, v[i].y, v[i].z, v[i].w);
   }
+  __device__ __forceinline__ float largest(float m) const {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) m = s3_largest(m, v[i]);
+    return m;
+  }
 };
 
 // MN-contiguous operand of R rows (element (row, k) at p[k ld + row]): a
@@ -136,7 +156,7 @@ struct S3K {
 // past krem read zero.
 template <int R>
 struct S3M {
-  float4 v[4];
+  float4 v[4] = {};  // (zero in the waves that load nothing)
   __device__ __forceinline__ void load(const float* p, int64_t ld, int64_t cols, int64_t krem) {
     const int lane = threadIdx.x & 63, w = wave_id();
     if (w >= R / 32) return;
@@ -157,6 +177,11 @@ struct S3M {
     s3_put<R * 64>(op + (a ^ 64u), v[0].y, v[1].y, v[2].y, v[3].y);
     s3_put<R * 64>(op + (a ^ 128u), v[0].z, v[1].z, v[2].z, v[3].z);
     s3_put<R * 64>(op + (a ^ 192u), v[0].w, v[1].w, v[2].w, v[3].w);
+  }
+  __device__ __forceinline__ float largest(float m) const {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) m = s3_largest(m, v[j]);
+    return m;
   }
 };
 
@@ -203,6 +228,61 @@ __device__ __forceinline__ void s3_mul(S3Acc<C::MB>& acc, const char* opA, const
         if constexpr (SWAP) c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[pb[t]][nb], a[pa[t]], c, 0, 0, 0);
         else c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[pa[t]], b[pb[t]][nb], c, 0, 0, 0);
       }
+  }
+}
+
+// The workgroup's marks, behind the second stage: mark i % 2 holds the last of
+// its tiles i, counted from 1, with a value past kS3Max.  A thread marks tile i
+// as it splits the tile's last step, a step before that is multiplied, and the
+// mark is read when it has been: a barrier lies between, and one more before
+// tile i + 2 writes there.
+struct S3Marks {
+  int* mark;
+  float big = 0.f;
+  __device__ __forceinline__ explicit S3Marks(char* p) : mark(reinterpret_cast<int*>(p)) {
+    if (threadIdx.x < 2) mark[threadIdx.x] = 0;
+    stage_barrier();
+  }
+  __device__ __forceinline__ void last_put(int tile) {
+    if (big > kS3Max) mark[tile & 1] = tile + 1;
+    big = 0.f;
+  }
+  __device__ __forceinline__ bool met(int tile) const {
+    return __builtin_amdgcn_readfirstlane(mark[tile & 1]) == tile + 1;
+  }
+};
+
+// The kernel's argument (its first), read where it is used: the rarely taken
+// code below would keep a dozen of its fields in SGPRs through the K loop.
+template <class P>
+__device__ __forceinline__ const __attribute__((address_space(4))) P* s3_args() {
+  uint64_t p = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return (const __attribute__((address_space(4))) P*)p;
+}
+
+// A wave's accumulators (blocks nb in [J0, J1)) += the products of k in [k0, k1)
+// on the native fp32 MFMA (16x16x4): av(mb, k) and bv(nb, k) are the operands'
+// values of the lane's row (lane % 16 of a block), from memory, zero outside it.
+template <class C, int J0, int J1, bool SWAP, class AV, class BV>
+__device__ __forceinline__ void s3_native(S3Acc<C::MB>& acc, int64_t k0, int64_t k1, const AV& av, const BV& bv) {
+  const int kl = opaque_lane() >> 4;
+#pragma unroll 1
+  for (; k0 < k1; k0 += 4) {
+    const int64_t k = k0 + kl;
+    float b[C::MB];
+#pragma unroll
+    for (int nb = J0; nb < J1; ++nb) b[nb] = k < k1 ? bv(nb, k) : 0.f;
+#pragma unroll
+    for (int mb = 0; mb < C::MB; ++mb) {
+      const float a = k < k1 ? av(mb, k) : 0.f;
+#pragma unroll
+      for (int nb = J0; nb < J1; ++nb) {
+        f32x4& c = acc[mb][nb];
+        if constexpr (SWAP) c = __builtin_amdgcn_mfma_f32_16x16x4f32(b[nb], a, c, 0, 0, 0);
+        else c = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b[nb], c, 0, 0, 0);
+      }
+    }
   }
 }
 
@@ -292,9 +372,16 @@ __global__ __launch_bounds__(C::kThreads, C::MB == 4 ? 2 : 3) void k_gemm_s3(Gem
       if (++fi < nt) f = tile_of(fi);
     }
   };
+  S3Marks marks(lds + 2 * C::kStage);
+  int pi = 0, ps = 0;  // tile and step being split
   auto put = [&](char* st) __attribute__((always_inline)) {
     la.store(st);
     lb.store(st + RA * 192);
+    marks.big = lb.largest(la.largest(marks.big));
+    if (++ps == steps) {
+      ps = 0;
+      marks.last_put(pi++);
+    }
   };
   const int w = wave_id(), wm = w >> 1, wn = w & 1;
   S3Acc<MB> acc;
@@ -308,6 +395,27 @@ __global__ __launch_bounds__(C::kThreads, C::MB == 4 ? 2 : 3) void k_gemm_s3(Gem
     ms = 0;
     const Tile x = tile_of(mi++);
     const int ol = opaque_lane();
+    if (P.K <= kS3Short || marks.met(mi - 1)) {
+      s3_zero<MB>(acc);
+      const auto* q = s3_args<GemmParams>();
+      const float* a = static_cast<const float*>(q->A);
+      const float* b = static_cast<const float*>(q->B);
+      const float* b1 = static_cast<const float*>(q->B1);
+      const int64_t kb = (int64_t)x.split * q->k_per_split, seg = b1 ? q->b_kseg : q->K;
+      const int64_t m = x.m0 + wm * 16 * MB + (ol & 15), n = x.n0 + wn * 16 * MB + (ol & 15);
+      auto av = [&](int mb, int64_t k) {
+        const int64_t r = m + mb * 16;
+        return r < q->M ? a[LA == KMAJ ? r * q->lda + k : k * q->lda + r] : 0.f;
+      };
+      auto bv = [&](int nb, int64_t k) {
+        const int64_t c = n + nb * 16;
+        if (c >= q->N) return 0.f;
+        if (LB == KMAJ) return b[c * q->ldb + k];
+        if (k >= seg) return k - seg < q->b_kval1 ? b1[(k - seg) * q->ldb1 + c] : 0.f;
+        return k < q->b_kval0 ? b[k * q->ldb + c] : 0.f;
+      };
+      s3_native<C, 0, MB, true>(acc, kb, min<int64_t>(q->K, b1 ? q->K : kb + q->k_per_split), av, bv);
+    }
     const int mlim = (int)min<int64_t>(P.M - x.m0, RA), nlim = (int)min<int64_t>(P.N - x.n0, RB);
     float* D = (MODE == GEMM_SPLIT || MODE == GEMM_ACC ? P.C32 + x.split * P.split_stride : static_cast<float*>(P.C)) + x.m0 * P.ldc + x.n0;
 #pragma unroll
@@ -360,6 +468,8 @@ struct S3MemAP {
 };
 template <> struct GuardMasked<S3PairAP> : std::true_type {};
 template <> struct GuardMasked<S3MemAP> : std::true_type {};
+template <> struct GuardStudent<S3PairAP> : std::true_type {};
+template <> struct GuardStudent<S3MemAP> : std::true_type {};
 
 // The lane's token's teacher logits at its rows of the tile, from [N x V]
 // memory or L's teacher columns (rows past V: unused).
@@ -453,11 +563,16 @@ __global__ __launch_bounds__(S3Big::kThreads, 2) void k_scan_s3(FusedParams P) {
       ++fv;
     }
   };
-  int ps = 0;  // step being split
+  S3Marks marks(lds + 2 * C::kStage);
+  int ps = 0, pv = 0;  // step and tile being split
   auto put = [&](char* sg) __attribute__((always_inline)) {
     la.store(sg);
     lb.store(sg + RA * 192 + (TS == S3_SEP && ps >= s0 ? 64 * 64 : 0));
-    if (++ps == steps) ps = 0;
+    marks.big = lb.largest(la.largest(marks.big));
+    if (++ps == steps) {
+      ps = 0;
+      marks.last_put(pv++);
+    }
   };
   S3Acc<MB> acc;
   s3_zero<MB>(acc);
@@ -476,6 +591,25 @@ __global__ __launch_bounds__(S3Big::kThreads, 2) void k_scan_s3(FusedParams P) {
     const int64_t vlimit = P.V - v0;
     const int ol = opaque_lane();  // (the epilogue's addresses stay out of the K loop's registers)
     const int vlane0 = wm * 64 + 4 * (ol >> 4);
+    if (P.H <= kS3Short || (TS == S3_SEP && P.Ht <= kS3Short) || marks.met(mv - 1 - vt0)) {
+      s3_zero<MB>(acc);
+      const auto* q = s3_args<FusedParams>();
+      auto rows = [&](const void* p, int64_t ld) {
+        return [=](int mb, int64_t k) {
+          const int64_t v = v0 + wm * 64 + mb * 16 + (ol & 15);
+          return v < q->V ? static_cast<const float*>(p)[v * ld + k] : 0.f;
+        };
+      };
+      auto cols = [&](const void* p, int64_t ld) {
+        return [=](int nb, int64_t k) {
+          const int64_t t = t0 + wcol + (PAIR ? nb & 1 : nb) * 16 + (ol & 15);
+          return t < q->N ? static_cast<const float*>(p)[t * ld + k] : 0.f;
+        };
+      };
+      s3_native<C, 0, PAIR ? 2 : 4, false>(acc, 0, q->H, rows(q->W, q->H), cols(q->hs, q->H));
+      if constexpr (TS == S3_TIED) s3_native<C, 2, 4, false>(acc, 0, q->H, rows(q->W, q->H), cols(q->ht, q->H));
+      if constexpr (TS == S3_SEP) s3_native<C, 2, 4, false>(acc, 0, q->Ht, rows(q->Wt, q->Ht), cols(q->ht, q->Ht));
+    }
     if constexpr (STORE) {
 #pragma unroll
       for (int nb = 0; nb < 4; ++nb) {
