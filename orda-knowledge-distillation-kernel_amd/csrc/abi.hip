@@ -70,8 +70,10 @@ constexpr int64_t kSplitTargetGroups = 512;
 // The ring engine addresses an MN-major operand's K range of one split as one
 // buffer resource whose record count is a 32-bit byte count.
 constexpr int64_t kRsrcBytes = 0x7fffffffll;
-// Largest hidden size (K-major rows of 128 x hidden x 4 bytes stay below 2^31)
-// and largest tokens per chunk (the chunk buffer's rows, 2 x chunk columns).
+// Largest hidden size (the 256 K-major rows that one buffer resource addresses
+// stay within its range, 2^32 bytes in the fp32 engine and 2^31 elsewhere; the
+// two-stage engine's fp32 rows at half of it) and largest tokens per chunk (the
+// chunk buffer's rows, 2 x chunk columns).
 constexpr int64_t kMaxHidden = 1ll << 22;
 constexpr int64_t kMaxChunkTokens = 1ll << 20;
 
@@ -385,6 +387,9 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
     kps = round_up(cdiv(pl.Vc, sp), 64);
     splits = (int)cdiv(pl.Vc, kps);
   };
+  if (f32 && !pl.fused && (pl.bwd_student || pl.bwd_teacher) &&
+      std::max(pl.H, pl.bwd_tsrc == TSRC_SEP ? pl.Ht : 0) > kMaxHidden / 2)
+    return fail(ORDA_EINVAL, "the two-phase backward in fp32 takes hidden sizes up to %lld", (long long)(kMaxHidden / 2));
   if (!pl.fused && pl.need_gs) bwd_split(pl.H, pl.bwd_splits_s, pl.bwd_kps_s);
   if (!pl.fused && pl.w_dln_t) bwd_split(pl.Ht, pl.bwd_splits_t, pl.bwd_kps_t);
   off = 0;

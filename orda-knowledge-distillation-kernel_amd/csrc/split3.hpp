@@ -108,7 +108,10 @@ __device__ __forceinline__ float4 s3_load(__amdgpu_buffer_rsrc_t rs, uint32_t of
   const u4v_t v = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0);
   return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
 }
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t s3_rsrc(const float* p) { return uniform_rsrc(p, 0x7fffffff); }
+// All but 16 of the 2^32 bytes that a resource can address: 256 K-major rows of
+// 2^22 values (the largest hidden size) stay below kS3Oob.
+constexpr uint32_t kS3Oob = 0xfffffff0u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t s3_rsrc(const float* p) { return uniform_rsrc(p, kS3Oob); }
 
 // (a NaN counts as nothing: its products are NaN on any path)
 __device__ __forceinline__ float s3_largest(float m, const float4& x) {
@@ -132,7 +135,7 @@ struct S3K {
     for (int i = I0; i < I1; ++i) {
       const int row = r + kStride * (i - I0);
       const bool ok = row < rows && kq * 4 < krem;
-      v[i] = s3_load(rs, ok ? (uint32_t)row * (uint32_t)(ld * 4) + (uint32_t)(kq * 16) : kOob);
+      v[i] = s3_load(rs, ok ? (uint32_t)row * (uint32_t)(ld * 4) + (uint32_t)(kq * 16) : kS3Oob);
     }
   }
   __device__ __forceinline__ void store(char* op) const {
@@ -165,7 +168,7 @@ struct S3M {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const bool ok = m0 < cols && k0 + j < krem;
-      v[j] = s3_load(rs, ok ? (uint32_t)(k0 + j) * (uint32_t)(ld * 4) + (uint32_t)(m0 * 4) : kOob);
+      v[j] = s3_load(rs, ok ? (uint32_t)(k0 + j) * (uint32_t)(ld * 4) + (uint32_t)(m0 * 4) : kS3Oob);
     }
   }
   __device__ __forceinline__ void store(char* op) const {

@@ -98,3 +98,24 @@ def test_vocabulary_rows_masked_by_an_infinite_bias(start, length, mode, w_t, tr
         cols = np.arange(H) != 7  # (the constant column's own gradient is 0 x -inf)
         got, want = _np(hs_d.grad)[:, cols], ref["grad_student_hidden"][:, cols]
         assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
+
+
+def test_hidden_rows_past_two_gigabytes_of_a_tile():
+    """256 vocabulary rows of 3 x 2^20 fp32 values are 3 GiB: every row counts.
+    The products' magnitudes sum to 1.1e3, of which a long fp32 sum is off by
+    2.5e-8 and more (2.8e-5 per logit); rows read as zero move the CE by 0.1."""
+    o = _orda()
+    N, H, V = 5, 3 << 20, 300
+    g = torch.Generator(device="cuda").manual_seed(4)
+    h = torch.randn(N, H, generator=g, device="cuda")
+    W = torch.randn(V, H, generator=g, device="cuda").mul_(H ** -0.5)
+    y = torch.tensor([255, 3, 299, 180, 140], device="cuda")
+    lt = torch.randn(N, V, generator=g, device="cuda")
+    with torch.no_grad():
+        out = o.distillation_loss(h, W, y, o.PrecomputedTeacher(logits=lt), kl_weight=0.5, backend="hip")
+    x = torch.cat([h.double() @ W[v:v + 50].double().t() for v in range(0, V, 50)], 1)
+    logp, logt = torch.log_softmax(x, -1), torch.log_softmax(lt.double(), -1)
+    ce = -logp.gather(1, y[:, None]).mean()
+    kl = (logt.exp() * (logt - logp)).sum(-1).mean()
+    assert abs(float(out.student_ce) - float(ce)) <= 4e-4
+    assert abs(float(out.kl) - float(kl)) <= 4e-4

@@ -57,3 +57,15 @@ def test_two_phase_workspace_holds_one_fp32_sum(N, H, V):
     p = _problem(N=N, H=H, V=V, flags=GRADS)
     got = _native.backward_workspace_bytes(p)
     assert got <= 4 * N * H + 2 * 2 * N * H + (512 << 20) + (1 << 20), got / 2 ** 20
+
+
+def test_fp32_hidden_sizes_past_a_resource():
+    """2^22 for the split-operand engine (256 rows in a resource of 4 GiB); the
+    two-phase backward's two-stage kernel has 2 GiB, so half of that."""
+    wide = dict(dtype=F32, N=64, H=1 << 22, V=1024)
+    assert _native.forward_workspace_bytes(_problem(flags=("compute_divergence",), **wide)) > 0
+    assert _native.forward_workspace_bytes(_problem(flags=GRADS + ("grads_in_forward",), **wide)) > 0
+    with pytest.raises(ValueError, match="two-phase"):
+        _native.forward_workspace_bytes(_problem(flags=GRADS, **wide))
+    wide["H"] = 1 << 21
+    assert _native.backward_workspace_bytes(_problem(flags=GRADS, **wide)) > 0
