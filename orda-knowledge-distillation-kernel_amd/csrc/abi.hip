@@ -390,6 +390,12 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
   if (f32 && !pl.fused && (pl.bwd_student || pl.bwd_teacher) &&
       std::max(pl.H, pl.bwd_tsrc == TSRC_SEP ? pl.Ht : 0) > kMaxHidden / 2)
     return fail(ORDA_EINVAL, "the two-phase backward in fp32 takes hidden sizes up to %lld", (long long)(kMaxHidden / 2));
+  // grad W reads the staged dlogits (and in 16 bits the transposed hidden states)
+  // K-major: 128 (fp32: 256) rows of ldT tokens from one buffer resource
+  if (!pl.fused && (pl.need_gw || pl.w_dlt_t) &&
+      pl.ldT * pl.eb > (f32 ? 0xfffffff0ll / 256 : kRsrcBytes / 128))
+    return fail(ORDA_EINVAL, "the two-phase backward's weight gradient takes up to %lld tokens (with teacher CE half of that)",
+                (long long)((f32 ? 0xfffffff0ll / 256 : kRsrcBytes / 128) / pl.eb / 8 * 8));
   if (!pl.fused && pl.need_gs) bwd_split(pl.H, pl.bwd_splits_s, pl.bwd_kps_s);
   if (!pl.fused && pl.w_dln_t) bwd_split(pl.Ht, pl.bwd_splits_t, pl.bwd_kps_t);
   off = 0;

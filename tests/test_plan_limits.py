@@ -29,7 +29,8 @@ GRADS = ("need_grad_student_hidden", "need_grad_weight", "compute_teacher_ce", "
     (BF16, 1 << 23, 64, 4096, GRADS + ("grads_in_forward",)), (F32, 1 << 22, 64, 4096, GRADS + ("grads_in_forward",)),
     (BF16, (1 << 24) + 64, 64, 4096, ("compute_divergence",)), (F32, (1 << 23) + 64, 64, 4096, ("compute_divergence",)),
     (BF16, 1 << 30, 64, 4096, ()), (BF16, 64, 131072, 600000, ("compute_divergence",)),
-    (BF16, 64, 131072, 600000, GRADS), (F32, 64, 131072, 600000, GRADS), (F16, (1 << 24) + 64, 64, 4096, GRADS),
+    (BF16, 64, 131072, 600000, GRADS), (F32, 64, 131072, 600000, GRADS),
+    (F16, (1 << 24) + 64, 64, 4096, ("need_grad_student_hidden",)),
     (BF16, 64, 131072, 600000, ("need_grad_weight",))])
 def test_large_calls_are_planned(dtype, N, H, V, flags):
     """A limit of the grad-hidden GEMM's split ranges does not refuse calls that
@@ -69,3 +70,16 @@ def test_fp32_hidden_sizes_past_a_resource():
         _native.forward_workspace_bytes(_problem(flags=GRADS, **wide))
     wide["H"] = 1 << 21
     assert _native.backward_workspace_bytes(_problem(flags=GRADS, **wide)) > 0
+
+
+@pytest.mark.parametrize("dtype,most", [(BF16, 8388600), (F16, 8388600), (F32, 4194296)])
+def test_two_phase_weight_gradient_of_too_many_tokens_is_refused(dtype, most):
+    """Its K-major rows of tokens stay inside a buffer resource; past it they
+    would wrap around."""
+    flags = ("need_grad_weight", "compute_divergence")
+    assert _native.backward_workspace_bytes(_problem(dtype=dtype, N=most, H=64, V=512, flags=flags)) > 0
+    with pytest.raises(ValueError, match="tokens"):
+        _native.forward_workspace_bytes(_problem(dtype=dtype, N=most + 1, H=64, V=512, flags=flags))
+    with pytest.raises(ValueError, match="tokens"):
+        _native.forward_workspace_bytes(_problem(dtype=dtype, N=most // 2 + 8, H=64, V=512,
+                                                 flags=flags + ("compute_teacher_ce",)))
