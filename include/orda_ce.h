@@ -230,7 +230,8 @@ typedef struct orda_plan_info {
   int32_t grads_in_forward;      /* 1: gradients-in-forward schedule          */
   int32_t table_entry;           /* launch-table row used, -1 = rule          */
   int32_t teacher_class;         /* 0 tied, 1 staged, 2 in place, 3 other     */
-  int32_t scan_engine;           /* 0 two-stage (8 waves), 1 ring (4 waves)   */
+  int32_t scan_engine;           /* 0 two-stage (8 waves), 1 ring (4 waves),
+                                    2 split-operand (fp32)                    */
   int64_t token_chunk;           /* tokens per chunk                          */
   int64_t n_token_chunks;
   int32_t chunk_scale;           /* token_chunk / requested chunk             */

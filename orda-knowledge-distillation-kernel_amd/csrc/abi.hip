@@ -85,7 +85,7 @@ struct Plan {
   float pa[3], pb[3];
   // forward
   bool fwd_ring;
-  int f_tok, n_ttiles, n_vtiles, n_vranges, tiles_per_range;
+  int f_tok, fwd_tok, n_ttiles, n_vtiles, n_vranges, tiles_per_range;  // (tokens per scan tile: f_tok of a chunk's)
   size_t off_partial, off_labelx, off_rowv, fwd_bytes;
   size_t saved_bytes;
   // backward
@@ -322,7 +322,6 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
   // forward plan.  Scan tiles of 256 vocabulary rows x 128 tokens; fp32: 64
   // tokens when the tile also holds a teacher's GEMM.
   const bool f32 = p->dtype == ORDA_F32;
-  pl.n_ttiles = (int)cdiv(pl.N, f32 && (pl.tsrc == TSRC_SHARED || pl.tsrc == TSRC_SEP) ? 64 : 128);
   pl.n_vtiles = (int)cdiv(pl.V, 256);
   // 16-bit without a teacher's GEMM beside the student's: the ring engine's
   // student-only tiles of 256 tokens, teacher logits of the compute dtype read
@@ -333,7 +332,8 @@ int make_plan(const orda_problem_t* p, Plan& pl) {
   const bool ring_mem = pl.tsrc == TSRC_MEM && p->logits_dtype == p->dtype && pl.V % 4 == 0 &&
                         pl.V <= 65535 * 64 && !(pl.fam == FAM_POW && pl.npow != 1);
   pl.fwd_ring = !f32 && pl.H > 64 && (pl.tsrc == TSRC_NONE || ring_mem);
-  if (pl.fwd_ring) pl.n_ttiles = (int)cdiv(pl.N, 256);
+  pl.fwd_tok = pl.fwd_ring ? 256 : f32 && (pl.tsrc == TSRC_SHARED || pl.tsrc == TSRC_SEP) ? 64 : 128;
+  pl.n_ttiles = (int)cdiv(pl.N, pl.fwd_tok);
   int64_t nvr = (f32 || pl.fwd_ring) ? kPersistentGroups / pl.n_ttiles : cdiv(kScanTargetGroups, pl.n_ttiles);  // two-phase scan
   if (nvr < 1) nvr = 1;
   if (nvr > pl.n_vtiles) nvr = pl.n_vtiles;
@@ -1445,25 +1445,25 @@ int orda_plan_info(const orda_problem_t* p, orda_plan_info_t* out) {
   out->vocab_chunk = pl.Vc;
   out->forward_workspace_bytes = pl.fwd_bytes;
   out->backward_workspace_bytes = pl.bwd_bytes;
+  // the ring scan runs 16-bit tied teachers, teacher logits from memory (all but
+  // three-term power families) and 16-bit scans with no teacher; fp32 the
+  // split-operand engine; the rest the two-stage engine
+  const bool tied_ring = pl.tsrc == TSRC_SHARED && pl.eb == 2 && pl.H > 64;
+  const bool ring = tied_ring || (pl.fused ? pl.f_tl || pl.f_sring : pl.fwd_ring);
+  out->scan_engine = pl.eb == 4 ? 2 : ring ? 1 : 0;
   if (pl.fused) {
-    // the ring scan runs 16-bit tied teachers (two tokens per lane), teacher
-    // logits from memory of the non-power families and 16-bit scans with no
-    // teacher (four tokens per lane); the rest the two-stage engine
-    const bool ring = pl.tclass == TC_TIED || pl.f_tl || pl.f_sring;
-    out->scan_engine = ring ? 1 : 0;
     out->token_chunk = pl.fn;
     out->n_token_chunks = pl.fnchunks;
     out->chunk_scale = pl.chunk_scale;
-    out->scan_tokens_per_tile = (pl.f_tl || pl.f_sring) ? 256 : 128;
-    out->scan_workgroups = (int)(cdiv(pl.fn, out->scan_tokens_per_tile) * pl.f_nvr);
+    out->scan_tokens_per_tile = pl.f_tok;
+    out->scan_workgroups = (int)(cdiv(pl.fn, pl.f_tok) * pl.f_nvr);
     out->grad_hidden_splits = pl.splits_s;
     out->grad_teacher_hidden_splits = pl.splits_t;
     out->vocab_rows_per_split = pl.kps_s;
   } else {
-    out->scan_engine = 0;
     out->token_chunk = pl.N;
     out->n_token_chunks = 1;
-    out->scan_tokens_per_tile = 128;
+    out->scan_tokens_per_tile = pl.fwd_tok;
     out->scan_workgroups = pl.n_ttiles * pl.n_vranges;
   }
   return ORDA_OK;

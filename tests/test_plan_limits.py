@@ -83,3 +83,23 @@ def test_two_phase_weight_gradient_of_too_many_tokens_is_refused(dtype, most):
     with pytest.raises(ValueError, match="tokens"):
         _native.forward_workspace_bytes(_problem(dtype=dtype, N=most // 2 + 8, H=64, V=512,
                                                  flags=flags + ("compute_teacher_ce",)))
+
+
+TIED = ("compute_teacher_ce", "compute_divergence")
+STUDENT_GRADS = ("need_grad_student_hidden", "need_grad_weight", "grads_in_forward")
+
+
+# (workgroups: token tiles times vocabulary ranges of whole 256-row tiles, as
+# many ranges as keep them within 256 -- 2048 for the two-stage forward)
+@pytest.mark.parametrize("mode,dtype,N,H,V,flags,engine,tokens,groups", [
+    ("tied", F32, 512, 256, 4096, TIED + STUDENT_GRADS, 2, 64, 8 * 16),
+    ("tied", F32, 512, 256, 4096, TIED, 2, 64, 8 * 16), ("separate", F32, 512, 256, 4096, TIED, 2, 64, 8 * 16),
+    ("separate", F32, 512, 256, 4096, ("compute_divergence",) + STUDENT_GRADS, 2, 128, 4 * 16),
+    ("precomputed_logits", F32, 512, 256, 4096, ("compute_divergence",), 2, 128, 4 * 16),
+    ("tied", BF16, 4096, 4096, 128256, (), 1, 256, 16 * 16), ("tied", BF16, 4096, 64, 4096, (), 0, 128, 32 * 16),
+    ("tied", BF16, 512, 4096, 4096, TIED, 1, 128, 4 * 16), ("separate", F16, 512, 256, 4096, TIED, 0, 128, 4 * 16),
+    ("precomputed_logits", F16, 512, 256, 4096, ("compute_divergence",), 1, 256, 2 * 16),
+    ("precomputed_logits", F16, 512, 256, 4098, ("compute_divergence",), 0, 128, 4 * 17)])
+def test_plan_info_names_the_scan_that_runs(mode, dtype, N, H, V, flags, engine, tokens, groups):
+    info = _native.plan_info(_problem(mode, dtype, N, H, V, flags=flags))
+    assert (info["scan_engine"], info["scan_tokens_per_tile"], info["scan_workgroups"]) == (engine, tokens, groups)
