@@ -29,6 +29,7 @@ from dataclasses import dataclass
 
 import torch
 import torch.nn.functional as F
+from torch.autograd.forward_ad import unpack_dual
 
 from .. import _native
 from .._runtime import HAS_NATIVE, native_error
@@ -53,10 +54,13 @@ def without_autograd(*tensors):
     recording is off.  Inside ``Function.forward`` a parameter still says
     ``requires_grad`` under ``torch.no_grad()``, so an evaluation pass would
     compute every gradient and drop it (4096 tokens, hidden 4096, vocabulary
-    128256, tied: 14.0 ms against 6.6 for the forward-only scan)."""
+    128256, tied: 14.0 ms against 6.6 for the forward-only scan).  A tensor
+    with a forward-mode tangent stays as it is: the Functions have no jvp, and
+    autograd refuses it, where ``detach`` would drop the tangent."""
     if torch.is_grad_enabled():
         return tensors
-    return tuple(t.detach() if isinstance(t, torch.Tensor) else t for t in tensors)
+    return tuple(t.detach() if isinstance(t, torch.Tensor) and t.requires_grad and unpack_dual(t).tangent is None
+                 else t for t in tensors)
 
 
 def vocab_chunk_for(BT: int, V: int, chunk_size, max_chunks) -> int:

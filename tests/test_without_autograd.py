@@ -3,7 +3,9 @@
 own tensors are left as they are (CPU)."""
 from __future__ import annotations
 
+import pytest
 import torch
+import torch.autograd.forward_ad as fwd
 
 from orda_ce_kernel.ops._engine import without_autograd
 
@@ -18,3 +20,22 @@ def test_tensors_are_detached_only_when_recording_is_off():
     with torch.inference_mode():
         (d,) = without_autograd(w)
     assert not d.requires_grad and d.data_ptr() == w.data_ptr()
+
+
+@pytest.mark.parametrize("requires_grad", [False, True])
+def test_forward_mode_tangents_are_still_refused(requires_grad):
+    """A Function without a jvp refuses dual tensors; so it does after this."""
+    class Sum(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            return x.sum()
+
+        @staticmethod
+        def backward(ctx, g):
+            return g
+
+    x = torch.randn(3, requires_grad=requires_grad)
+    with fwd.dual_level(), torch.no_grad():
+        (y,) = without_autograd(fwd.make_dual(x, torch.ones(3)))
+        with pytest.raises(NotImplementedError):
+            Sum.apply(y)
