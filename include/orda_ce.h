@@ -301,10 +301,11 @@ int orda_backward(const orda_problem_t* p, const orda_tensors_t* t,
 int orda_scale_gradient(int32_t dtype, void* grad, int64_t numel, const float* factor, void* stream);
 
 /* Plain C = A * B^T with A [M x K], B [N x K] (both K-contiguous) and C
- * [M x N] in `dtype`, fp32 accumulation (the engine behind every GEMM of the
- * path).  Exposed for tests and for callers that want the MFMA engine alone;
- * replaces nothing in the reference directly (it stands for the torch
- * matmuls at ops/tied_teacher.py:445,473,493). */
+ * [M x N] in `dtype`, fp32 accumulation, C of any column count and alignment
+ * (the two-stage engine of the fused kernels).  Exposed for tests and for
+ * callers that want the MFMA engine alone; replaces nothing in the reference
+ * directly (it stands for the torch matmuls at
+ * ops/tied_teacher.py:445,473,493). */
 int orda_gemm_abt(int32_t dtype, int64_t M, int64_t N, int64_t K,
                   const void* A, const void* B, void* C, void* stream);
 
@@ -314,8 +315,10 @@ int orda_gemm_abt(int32_t dtype, int64_t M, int64_t N, int64_t K,
  * ([N x K] or [K x N]).  C is [M x N] with leading dimension ldc.  splits > 1
  * splits K into that many fp32 partials summed in a fixed order; the
  * workspace must then hold splits * M * N floats (else it may be NULL).
- * Exposed for tests and callers that want the engine; it stands for the
- * torch matmuls of ops/tied_teacher.py:445,473,493, whose operands the
+ * Exposed for tests and callers that want the engines of the gradient GEMMs
+ * (fp32: the split-operand engine, except for an MN-major A with a K-major B and
+ * for N off 4); it stands for the torch matmuls of
+ * ops/tied_teacher.py:445,473,493, whose operands the
  * materialised path reads in both layouts. */
 int orda_gemm(int32_t dtype, int32_t a_mn, int32_t b_mn, int64_t M, int64_t N, int64_t K, const void* A,
               int64_t lda, const void* B, int64_t ldb, void* C, int64_t ldc, int32_t splits, void* workspace,

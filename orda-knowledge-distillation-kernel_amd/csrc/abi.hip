@@ -98,7 +98,8 @@ struct Plan {
   size_t off_hT, off_htT, off_dLT, off_bsplit, off_g32s, off_g32t, bwd_bytes;
   // gradients inside forward (materialised token chunks)
   bool fused, store_t, f_tl, f_tmem, f_sring, topk;
-  // fp16: dlogits without the mean scale, gradients scaled once at the end
+  // fp16: dlogits without the mean scale, which goes into each gradient's last
+  // rounding (behind the norm: one pass over its two)
   bool late_scale;
   int tclass, table_entry, chunk_scale, scan_groups;
   int64_t fn, fnP, fldL, fnchunks;

@@ -59,8 +59,8 @@ def without_autograd(*tensors):
     autograd refuses it, where ``detach`` would drop the tangent."""
     if torch.is_grad_enabled():
         return tensors
-    return tuple(t.detach() if isinstance(t, torch.Tensor) and t.requires_grad and unpack_dual(t).tangent is None
-                 else t for t in tensors)
+    return tuple([t.detach() if t is not None and t.requires_grad and unpack_dual(t).tangent is None else t
+                  for t in tensors])
 
 
 def vocab_chunk_for(BT: int, V: int, chunk_size, max_chunks) -> int:

@@ -1,9 +1,10 @@
 """The fp32 kernels (three-way bf16 split on the matrix cores) at the edges of
 their tiles, against the float64 oracle.
 
-Bound: an fp32 value is the exact sum of its three parts and the dropped
-products are below 2^-24 |a b|, so a dot product of K terms is off by at most
-(K / 32 + 6) 2^-24 sum |a b| (one rounding per 32-term MFMA and product).  With
+Bound: an fp32 value is the sum of its three parts and the dropped products are
+below 2^-24 |a b|, so a dot product of K terms is off by at most (6 K / 32 + 1)
+2^-24 sum |a b| (one rounding per 32-term MFMA and product; far less where the
+roundings' signs mix).  With
 K <= 600, logits of spread 1.5 and the softmax's exp on 2^-23 accurate
 hardware, losses and gradients agree to 1e-5 of their norm (1e-6 seen)."""
 from __future__ import annotations
