@@ -175,6 +175,11 @@ constexpr float kMaskedMax = -1e37f;
 template <class AP>
 struct GuardMasked : std::false_type {};
 template <> struct GuardMasked<AccPair2> : std::true_type {};
+// Guarded beside a FAM_LIN divergence too (losses only): its own sum is 0 times
+// a masked logit, NaN in any case, so only the teacher's CE is left to keep, and
+// the training scans of that family go without.
+template <class AP>
+struct GuardMaskedLin : std::false_type {};
 // The same for a lane's student logits: 16 rows per lane in fp32, whose logits
 // an infinite weight can mask.
 template <class AP>
@@ -188,8 +193,8 @@ __device__ __forceinline__ void scan_tile(RowState& S, const AP& acc, int vlane0
                                           const FusedParams& P) {
   // (the two-stage lanes' three power sums spill as it is, and multiply an
   // infinite logit by 0 anyway)
-  constexpr bool kGuard =
-      GuardMasked<AP>::value && !(std::is_same<AP, AccPair2>::value && FAM == FAM_POW && NPOW > 1);
+  constexpr bool kGuard = GuardMasked<AP>::value && (FAM != FAM_LIN || GuardMaskedLin<AP>::value) &&
+                          !(std::is_same<AP, AccPair2>::value && FAM == FAM_POW && NPOW > 1);
   const float invT = P.invT;
   float tms = -kInf, tmt = -kInf, tmu0 = -kInf, tmu1 = -kInf, tmu2 = -kInf;
 #pragma unroll
@@ -1260,7 +1265,7 @@ struct AccPair16S {  // student only: block j (the teacher accessor is never use
   __device__ __forceinline__ float s(int mb, int r) const { return acc16_get(a[mb][j], r); }
   __device__ __forceinline__ float t(int, int) const { return 0.f; }
 };
-template <class T>
+template <class T, bool STORE>
 struct AccPair16TL {  // student from block j, teacher from ordered raw registers
   using Lay = Layout16;
   const Acc16& a;
@@ -1273,9 +1278,10 @@ struct AccPair16TL {  // student from block j, teacher from ordered raw register
     return (r & 1) ? hi16<T>(w) : lo16<T>(w);
   }
 };
-template <class T> struct GuardMasked<AccPair16TL<T>> : std::true_type {};
-template <class T>
-__device__ __forceinline__ void acc_fence(const AccPair16TL<T>& p) {
+template <class T, bool STORE> struct GuardMasked<AccPair16TL<T, STORE>> : std::true_type {};
+template <class T> struct GuardMaskedLin<AccPair16TL<T, false>> : std::true_type {};
+template <class T, bool STORE>
+__device__ __forceinline__ void acc_fence(const AccPair16TL<T, STORE>& p) {
   uint2* r = const_cast<uint2*>(p.tr);
 #pragma unroll
   for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(r[i].x), "+v"(r[i].y));
@@ -1357,7 +1363,7 @@ __global__ __launch_bounds__(kThreads4, 1) void k_scan16(FusedParams P) {
         if constexpr (TL == TL_FROM_MEM && STORE) {
           if (P.store_t) store_teacher16<T>(raw[j & 1], P, x.v0, t0, j);  // else the dlogits pass reads them in place
         }
-        scan_variant<SV>(st[j], AccPair16TL<T>{c, j, raw[j & 1]}, vlane0, vlimit, vlimit >= 256, lse_sT[j],
+        scan_variant<SV>(st[j], AccPair16TL<T, STORE>{c, j, raw[j & 1]}, vlane0, vlimit, vlimit >= 256, lse_sT[j],
                          lse_tT[j], P);
         if (STORE && !full) store_block16<T>(c, P, x.v0, t0, j);
         if constexpr (j + 2 < NJ) issue_teacher16<T, TL>(raw[j & 1], P, x.v0, t0, j + 2);

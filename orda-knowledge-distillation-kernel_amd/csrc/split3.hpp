@@ -471,6 +471,8 @@ struct S3MemAP {
 };
 template <> struct GuardMasked<S3PairAP> : std::true_type {};
 template <> struct GuardMasked<S3MemAP> : std::true_type {};
+template <> struct GuardMaskedLin<S3PairAP> : std::true_type {};
+template <> struct GuardMaskedLin<S3MemAP> : std::true_type {};
 template <> struct GuardStudent<S3PairAP> : std::true_type {};
 template <> struct GuardStudent<S3MemAP> : std::true_type {};
 
