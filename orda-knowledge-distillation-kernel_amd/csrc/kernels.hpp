@@ -3302,7 +3302,7 @@ inline void gemm2_go(const GemmParams& P, hipStream_t s) {
       return;
     }
   }
-  if constexpr (sizeof(T) == 2 && LA == KMAJ && LB == MNMAJ && (MODE == GEMM_STORE || MODE == GEMM_ACC_T)) {
+  if constexpr (sizeof(T) == 2 && LA == KMAJ && LB == MNMAJ) {
     const int64_t lim = 0x7fffffffll / (int64_t)sizeof(T);
     if (P.splits == 1 && P.K > 64 && !P.B1 && P.b_kval0 * P.ldb < lim) {
       hipLaunchKernelGGL((k_gemm4<T, KMAJ, MNMAJ, MODE>), dim3(grid), dim3(kThreads4), 0, s, P);
@@ -3325,7 +3325,6 @@ inline void gemm2_go(const GemmParams& P, hipStream_t s) {
     using T = TYPE;                                                                        \
     switch (P.la * 100 + P.lb * 10 + P.mode) {                                             \
       ORDA_GEMM2_CASE(KMAJ, MNMAJ, GEMM_STORE)                                             \
-      ORDA_GEMM2_CASE(KMAJ, MNMAJ, GEMM_ACC_T)                                             \
       ORDA_GEMM2_CASE(MNMAJ, MNMAJ, GEMM_STORE)                                            \
       ORDA_GEMM2_CASE(MNMAJ, MNMAJ, GEMM_SPLIT)                                            \
       ORDA_GEMM2_CASE(MNMAJ, MNMAJ, GEMM_ACC)                                              \
