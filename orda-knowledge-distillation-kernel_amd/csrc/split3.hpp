@@ -1,11 +1,11 @@
 // fp32 GEMMs and scans on the bf16 matrix cores of gfx950.
 //
-// An fp32 value is the exact sum of three bf16 values, x = x1 + x2 + x3 (8 +
-// 8 + 8 significant bits: x1 and x2 rounded to nearest, so |x2| <= 2^-8 |x| and
-// |x3| <= 2^-17 |x|, either sign; x3 exact above 2^-109, below it off by at most
-// 2^-133), and a product
-// a b is taken as the six partial products a1 b1, a1 b2, a2 b1, a2 b2, a1 b3,
-// a3 b1, exact in the fp32 accumulators of v_mfma_f32_16x16x32_bf16; the three
+// An fp32 value is the sum of three bf16 values, x = x1 + x2 + x3 (8 + 8 + 8
+// significant bits: x1 and x2 rounded to nearest, so |x2| <= 2^-8 |x| and |x3|
+// <= 2^-17 |x|, either sign; exact above 2^-109, below it x3 is a bf16 subnormal,
+// off by at most 2^-133), and a product a b is taken as the six partial products
+// a1 b1, a1 b2, a2 b1, a2 b2, a1 b3, a3 b1, exact in the fp32 accumulators of
+// v_mfma_f32_16x16x32_bf16 (which keeps subnormal operands); the three
 // left out are below 2^-24 + 2^-34 of |a b|, of either sign.  The signs matter:
 // an MFMA drops bits of products far below its accumulator, and with x1
 // truncated (x2 of x's sign) a sum of 4096 positive products lost 3.6e-6 of its
@@ -16,7 +16,7 @@
 // Six bf16 products per fp32 one: 2500 / 6 = 417 TFLOP/s against the fp32
 // units' 157.  Measured against the native fp32 MFMA (32x32x2) kernels this
 // replaces: 170 against 110 TFLOP/s in the GEMMs; 1000 tokens, hidden 1000,
-// teacher hidden 1200, vocabulary 30001: 2.44 -> 1.50 ms a step, gradients off
+// teacher hidden 1200, vocabulary 30001: 2.44 -> 1.49 ms a step, gradients off
 // float64 by 6.4e-7 of their norm against 9e-7; 512 x 256 x 4096: 504 -> 128 us
 // of kernels.  All eight products down to 2^-34 take 1.70 ms for the former at
 // the same error.  The matrix cores are busy 56% of the cycles at 1.94 GHz (the

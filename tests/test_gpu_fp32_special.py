@@ -1,6 +1,7 @@
 """fp32 operands without a three-way bf16 split (infinities, magnitudes that
 round past the bf16 range) and short sums, where the split-operand engine takes
-the native fp32 MFMA: results as fp32 units give them."""
+the native fp32 MFMA: results as fp32 units give them.  And operands so small
+that their parts end in bf16's subnormals."""
 from __future__ import annotations
 
 import numpy as np
@@ -59,6 +60,21 @@ def test_infinite_and_huge_operands(M, N, K, splits):
         assert torch.equal(c[inf], exact[inf]), name
         err = ((c - exact).abs() / size)[fits & ~torch.isnan(exact)]
         assert float(err.max()) <= (K / 4 + 8) * 2.0 ** -24, (name, float(err.max()))
+
+
+@pytest.mark.parametrize("M,N", [(320, 384), (4096, 2048)])
+@pytest.mark.parametrize("exponent", [-100, -112, -120])
+def test_operands_with_parts_in_the_subnormal_range(exponent, M, N):
+    """Below 2^-109 the third part is a bf16 subnormal: each product is off by
+    2^-133 of the other operand at most, beside a sum's usual rounding."""
+    K = 64
+    a, b = _operands("normal", M, N, K)
+    a = a * 2.0 ** exponent
+    exact = a.double() @ b.double().t()
+    size = a.double().abs() @ b.double().abs().t()
+    bound = b.double().abs().sum(1) * 2.0 ** -133 + (6 * K / 32 + 1) * 2.0 ** -24 * size
+    for name, c in _layouts(a, b):
+        assert bool(((c.double() - exact).abs() <= bound).all()), name
 
 
 @pytest.mark.parametrize("train", [False, True])
